@@ -55,4 +55,9 @@ int launch_repack(int quant, const void* src, int64_t n_in, int64_t n_out, void*
 int launch_repack_experts(int quant, const void* src, int64_t n_in, int64_t n_rows, void* dst, int* dst_quant,
                           hipStream_t s);
 
+// y = W x from the f32 input in one launch (the input quantized by every workgroup); false, with
+// nothing launched, for the shapes that it does not take.  x: 16-byte aligned; arguments checked.
+bool launch_vec_dot_fused(int quant, const void* w, int64_t n_in, int64_t n_out, const float* x, float* y,
+                          hipStream_t s);
+
 }  // namespace jero

@@ -464,6 +464,21 @@ int launch_repack_experts(int quant, const void* src, int64_t n_in, int64_t n_ro
 
 using namespace jero;
 
+namespace {
+// y = W x for a quantized format: one launch where the fused kernel takes the shape, else the
+// quantizer into ws (an activation row) and the GEMV, which also serve an output that overlaps the
+// input (the fused launch's workgroups read the input while others write their rows).
+int launch_vec_dot(int act, int quant, const void* w, int64_t n_in, int64_t n_out, const float* x, void* ws, float* y,
+                   hipStream_t s) {
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+  const bool overlap = xa < ya + size_t(n_out) * 4 && ya < xa + size_t(n_in) * 4;
+  if (!overlap && launch_vec_dot_fused(quant, w, n_in, n_out, x, y, s)) return check_launch("vec_dot");
+  int rc = launch_quantize_act(act, x, 1, n_in, ws, s);
+  if (rc) return rc;
+  return launch_matvec(quant, w, n_in, n_out, ws, y, nullptr, s);
+}
+}  // namespace
+
 extern "C" int jero_hip_matvec(int quant, const void* w_dev, size_t w_bytes, int64_t n_in, int64_t n_out,
                                const void* xq_dev, float* y_dev, void* stream) {
   int rc = check_matvec_args(quant, w_dev, w_bytes, n_in, n_out, xq_dev, y_dev);
@@ -500,9 +515,7 @@ extern "C" int jero_hip_vec_dot(int quant, const void* w_dev, size_t w_bytes, in
     rc = workspace(need, &ws);
     if (rc) return rc;
   }
-  rc = launch_quantize_act(act, x_dev, 1, n_in, ws, s);
-  if (rc) return rc;
-  return launch_matvec(quant, w_dev, n_in, n_out, ws, y_dev, nullptr, s);
+  return launch_vec_dot(act, quant, w_dev, n_in, n_out, x_dev, ws, y_dev, s);
 }
 
 // ---- the allocation-free vec_dot: activation staging in a static device array ----
@@ -552,9 +565,7 @@ extern "C" int jero_hip_vec_dot_noalloc(int quant, const void* w_dev, size_t w_b
   void* ws = nullptr;
   rc = scratch_ptr(&ws);
   if (rc) return rc;
-  rc = launch_quantize_act(act, x_dev, 1, n_in, ws, s);
-  if (rc) return rc;
-  return launch_matvec(quant, w_dev, n_in, n_out, ws, y_dev, nullptr, s);
+  return launch_vec_dot(act, quant, w_dev, n_in, n_out, x_dev, ws, y_dev, s);
 }
 
 extern "C" int jero_hip_repack(int quant, const void* src_dev, size_t src_bytes, int64_t n_in, int64_t n_out,
