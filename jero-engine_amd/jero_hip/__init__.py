@@ -153,14 +153,25 @@ def check(status):
         raise K3Error(status, msg)
 
 
+# Every pointer argument is a plain integer (the entry points' argtypes convert it), and the current
+# stream is read as its handle: a torch.cuda.Stream object per call cost as much as the launch's own
+# host work.
+_raw_stream = None
+
+
 def _stream(stream=None):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    global _raw_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()  # the first use initializes torch's GPU state
+        _raw_stream = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+    return _raw_stream[0](_raw_stream[1]())
 
 
 def _ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def init(device=0):
@@ -191,7 +202,7 @@ class TensorView:
         return self.shape[1] if len(self.shape) > 1 else 1
 
     def nbytes(self):
-        return self.data.numel() * self.data.element_size()
+        return self.data.nbytes
 
     def slice_rows(self, start, count):
         rb = row_bytes(self.quant, self.n_in)
@@ -492,8 +503,8 @@ def dispatch_qwen3_moe_ffn(out, norm_ffn_in, router_logits, top_k, gate, up, dow
     T = router_logits.shape[0] if router_logits.dim() == 2 else 1
     E = router_logits.shape[-1]
     hidden, ffn = gate.shape[0], gate.shape[1]
-    sel_idx = torch.empty((T, top_k), dtype=torch.int32, device=out.device)
-    sel_w = torch.empty((T, top_k), dtype=torch.float32, device=out.device)
+    sel_idx = out.new_empty((T, top_k), dtype=torch.int32)
+    sel_w = out.new_empty((T, top_k), dtype=torch.float32)
     if workspace is None:
         need = lib().jero_hip_moe_workspace_bytes(T, E, top_k, hidden, ffn)
         workspace = torch.empty(need, dtype=torch.uint8, device=out.device)
