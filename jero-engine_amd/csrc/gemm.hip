@@ -73,20 +73,20 @@ __device__ __forceinline__ void gemm_tile_of(int wg, int n_wg, int n_tiles_m, in
   tm = l % n_tiles_m;
 }
 
-// Every load is unconditional (rows past M read row M-1 and are never stored).  PLANAR: the weight
+// Every load is unconditional (rows past M or N read the last row and are never stored).  PLANAR: the weight
 // rows are in the Q4_K_R layout (each row's q0 run of U = 4 nb 16-byte pieces, its q1 run, then
 // its nb block headers); the chunks land in LDS as the same raw Q4_K block, so the rest of the
 // kernel, and its results, do not depend on the layout.
 template <bool PLANAR>
 __device__ __forceinline__ void q4k_load(Q4kRegs& R, const uint8_t* __restrict__ x, int64_t xrb, int m0, int M,
-                                         const uint8_t* __restrict__ w, int64_t wrb, int n0, int b, int nb) {
+                                         const uint8_t* __restrict__ w, int64_t wrb, int n0, int N, int b, int nb) {
   const int t = threadIdx.x, r = t >> 2, q = t & 3;
   const int m = min(m0 + r, M - 1);
   const uint8_t* xa = x + int64_t(m) * xrb + int64_t(b) * 292;
 #pragma unroll
   for (int i = 0; i < 4; i++) R.aq[i] = ld4(xa + 4 + 64 * q + 16 * i);
   R.ax = ld4(xa + (q == 1 ? 260 : q == 2 ? 276 : 0));
-  const uint8_t* rp = w + int64_t(n0 + r) * wrb;
+  const uint8_t* rp = w + int64_t(min(n0 + r, N - 1)) * wrb;
   // 16-byte chunk c of the row's block b: 0 = header, 1 + i = qs bytes [16 i, 16 i + 16)
   auto chunk = [&](int c) -> const uint8_t* {
     if constexpr (!PLANAR) {
@@ -152,12 +152,12 @@ __global__ void __launch_bounds__(kQ4Threads) gemm_q4k_kernel(const uint8_t* __r
     for (int v = 0; v < 16; v++) acc[i][v] = 0.f;
 
   Q4kRegs R;
-  q4k_load<PLANAR>(R, x, xrb, m0, M, w, wrb, n0, b0, nb);
+  q4k_load<PLANAR>(R, x, xrb, m0, M, w, wrb, n0, N, b0, nb);
   q4k_store(R, S[0]);
   __syncthreads();
   for (int b = b0; b < b1; b++) {
     const Q4kStage& T = S[(b - b0) & 1];
-    if (b + 1 < b1) q4k_load<PLANAR>(R, x, xrb, m0, M, w, wrb, n0, b + 1, nb);
+    if (b + 1 < b1) q4k_load<PLANAR>(R, x, xrb, m0, M, w, wrb, n0, N, b + 1, nb);
     // this lane's weight row: header d, dmin and the 6-bit scales / mins (GGUF Q4_K packing)
     const u32x4 hd = *reinterpret_cast<const u32x4*>(&T.w[nl][0]);
     uint32_t scv[8], mvv[4];
@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(kQ4Threads) gemm_q4k_kernel(const uint8_t* __r
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       const int m = m0 + 64 * wm + 32 * mt + 8 * (v >> 2) + 4 * lh + (v & 3);
-      if (m < M) {
+      if (m < M && n < N) {
         if constexpr (SPLIT) atomicAdd(&y[int64_t(m) * N + n], acc[mt][v]);
         else y[int64_t(m) * N + n] = acc[mt][v];
       }
@@ -806,6 +806,185 @@ __global__ void __launch_bounds__(kGpThreads, 2) gemm_laid_kernel(const uint8_t*
     }
 }
 
+// ---- Few tokens: K split over the waves of a workgroup.
+// Below a full grid of 64 x 128 tiles gemm_laid_kernel is bound by the serial chain of its blocks on
+// the few CUs that it reaches (37 tokens x 4096 rows: 64 workgroups, halves of K included, 42 us for
+// 24 blocks each).  Here a workgroup owns one 32-row record tile and 32 tokens, and each of its KW
+// waves walks its own run of the blocks alone: its record and its block's activations in registers
+// one block ahead, the activations through LDS of its own (a wave's LDS operations are in order: no
+// barrier in the loop).  The waves' f32 sums meet once, in LDS, added in wave order, so no zeroed
+// output, atomics or second buffer are needed.  What bounds it then is the record stream (Q6_K_P,
+// 2 bytes a weight) and, with more tokens, the re-reads: every 32-token tile reads all records and
+// every record tile all activations.  A 64-token tile per wave spilled or left one wave per SIMD
+// (37 x 4096 -> 1024 Q4_K_G: 13.7 us against 9.0).
+struct __attribute__((aligned(16))) KwStage {
+  int8_t a[32][kPlaneStride];
+  _Float16 bs[32][16];
+  float dx[32];
+};
+
+// A lane's share of one activation block of a wave's 32 token rows: piece lane % 16 of rows
+// 4 i + lane / 16, half lane % 2 of the bsums of row lane / 2, the d of row lane % 32.
+template <bool BSUMS>
+struct KwAct {
+  u32x4 q[8];
+  u32x4 bs;
+  uint32_t d;
+};
+
+template <bool BSUMS>
+__device__ __forceinline__ void kw_load_act(KwAct<BSUMS>& A, const uint8_t* __restrict__ xq, int64_t xrb, int m0,
+                                            int M, int b, int lane) {
+  const uint8_t* xb = xq + int64_t(b) * 292;
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    A.q[i] = ld4(xb + int64_t(min(m0 + 4 * i + (lane >> 4), M - 1)) * xrb + 4 + 16 * (lane & 15));
+  if constexpr (BSUMS) A.bs = ld4(xb + int64_t(min(m0 + (lane >> 1), M - 1)) * xrb + 260 + 16 * (lane & 1));
+  A.d = ld1(xb + int64_t(min(m0 + (lane & 31), M - 1)) * xrb);
+}
+
+template <bool BSUMS>
+__device__ __forceinline__ void kw_store_act(const KwAct<BSUMS>& A, KwStage& S, int lane) {
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    *reinterpret_cast<u32x4*>(&S.a[4 * i + (lane >> 4)][16 * (lane & 15)]) = A.q[i];
+  if constexpr (BSUMS) {
+    uint32_t hw[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      hw[i] = uint32_t(__builtin_bit_cast(uint16_t, _Float16(float(int16_t(A.bs[i] & 0xFFFFu))))) |
+              (uint32_t(__builtin_bit_cast(uint16_t, _Float16(float(int16_t(A.bs[i] >> 16))))) << 16);
+    *reinterpret_cast<u32x4*>(&S.bs[lane >> 1][8 * (lane & 1)]) = u32x4{hw[0], hw[1], hw[2], hw[3]};
+  }
+  S.dx[lane & 31] = __uint_as_float(A.d);
+}
+
+template <bool Q4, int KW>
+__global__ void __launch_bounds__(64 * KW, 8 / KW) gemm_laid_kw_kernel(const uint8_t* __restrict__ xq, int64_t xrb,
+                                                                        const uint8_t* __restrict__ wg, int M, int N,
+                                                                        int nb, float* __restrict__ y) {
+  static_assert(sizeof(KwStage) >= 16 * 64 * sizeof(float), "the waves' sums fit their stages");
+  __shared__ KwStage S[KW];
+  constexpr int REC = Q4 ? kQ4gRec : kQ6pRec;
+  int tm, tn;
+  gemm_tile_of(int(blockIdx.x), int(gridDim.x), (M + 31) / 32, tm, tn);
+  const int m0 = tm * 32;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lr = lane & 31, lh = lane >> 5;
+  const int b0 = nb * wv / KW, b1 = nb * (wv + 1) / KW;
+  const uint8_t* wt = wg + int64_t(tn) * nb * REC;
+  const uint8_t* wl = wt + 16 * lane;
+  const uint8_t* wr = wt + (Q4 ? 4096 + 16 * lane : kQ6pPlanes + 4 * lr);
+  KwStage& T = S[wv];
+
+  float acc[16];
+#pragma unroll
+  for (int v = 0; v < 16; v++) acc[v] = 0.f;
+
+  if (b0 < b1) {
+    KwAct<Q4> A;
+    constexpr int NW = Q4 ? 4 : 16;
+    u32x4 W[NW];
+    u32x4 H = {0u, 0u, 0u, 0u};
+    float dq = 0.f;
+    kw_load_act<Q4>(A, xq, xrb, m0, M, b0, lane);
+#pragma unroll
+    for (int i = 0; i < NW; i++) W[i] = ld4(wl + int64_t(b0) * REC + 1024 * i);
+    if constexpr (Q4) H = ld4(wr + int64_t(b0) * REC);
+    else dq = __uint_as_float(ld1(wr + int64_t(b0) * REC));
+    for (int b = b0; b < b1; b++) {
+      const int bn = min(b + 1, b1 - 1);  // the last block reloads itself: every load unconditional
+      const int64_t on = int64_t(bn) * REC;
+      kw_store_act<Q4>(A, T, lane);
+      __builtin_amdgcn_wave_barrier();
+      kw_load_act<Q4>(A, xq, xrb, m0, M, bn, lane);
+      float dw, dm = 0.f;
+      v8h mnf = {};
+      v16i Ch, Cl;
+      if constexpr (Q4) {
+        const u32x4 Hc = H;
+        H = ld4(wr + on);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) mnf[2 * jj] = mnf[2 * jj + 1] = _Float16(float(byte_of(Hc.w, jj)));
+        dw = float(__builtin_bit_cast(_Float16, uint16_t(Hc.x & 0xFFFFu)));
+        dm = float(__builtin_bit_cast(_Float16, uint16_t(Hc.x >> 16)));
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const uint32_t sw = i < 2 ? Hc.y : Hc.z;
+          const uint32_t s0 = byte_of(sw, 2 * (i & 1)), s1 = byte_of(sw, 2 * (i & 1) + 1);
+          const uint32_t raw[4] = {W[i].x, W[i].y, W[i].z, W[i].w};
+          W[i] = ld4(wl + on + 1024 * i);
+          v4i pa0, pb0, pa1, pb1;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const uint32_t ql = raw[e] & 0x0F0F0F0Fu, qh = (raw[e] >> 4) & 0x0F0F0F0Fu;
+            pa0[e] = int(pk_mul(ql, s0 >> 3));
+            pb0[e] = int(pk_mul(ql, s0 & 7u));
+            pa1[e] = int(pk_mul(qh, s1 >> 3));
+            pb1[e] = int(pk_mul(qh, s1 & 7u));
+          }
+          const v4i af0 = *reinterpret_cast<const v4i*>(&T.a[lr][64 * i + 16 * lh]);
+          const v4i af1 = *reinterpret_cast<const v4i*>(&T.a[lr][64 * i + 32 + 16 * lh]);
+          const v16i z = {};
+          Ch = __builtin_amdgcn_mfma_i32_32x32x32_i8(af0, pa0, i == 0 ? z : Ch, 0, 0, 0);
+          Cl = __builtin_amdgcn_mfma_i32_32x32x32_i8(af0, pb0, i == 0 ? z : Cl, 0, 0, 0);
+          Ch = __builtin_amdgcn_mfma_i32_32x32x32_i8(af1, pa1, Ch, 0, 0, 0);
+          Cl = __builtin_amdgcn_mfma_i32_32x32x32_i8(af1, pb1, Cl, 0, 0, 0);
+        }
+      } else {
+        __builtin_amdgcn_sched_barrier(0);
+        dw = dq;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+          const v4i af = *reinterpret_cast<const v4i*>(&T.a[lr][32 * s + 16 * lh]);
+          const v16i z = {};
+          Ch = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, __builtin_bit_cast(v4i, W[2 * s]), s == 0 ? z : Ch, 0, 0, 0);
+          Cl = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, __builtin_bit_cast(v4i, W[2 * s + 1]), s == 0 ? z : Cl, 0, 0,
+                                                     0);
+          W[2 * s] = ld4(wl + on + (2 * s) * 1024);
+          W[2 * s + 1] = ld4(wl + on + (2 * s + 1) * 1024);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        dq = __uint_as_float(ld1(wr + on));
+      }
+      v16f Mn = {};
+      if constexpr (Q4) {
+        const v8h bsf = *reinterpret_cast<const v8h*>(&T.bs[lr][8 * lh]);
+        Mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, mnf, Mn, 0, 0, 0);
+      }
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const float4 dx = *reinterpret_cast<const float4*>(&T.dx[8 * g + 4 * lh]);
+        const float dxv[4] = {dx.x, dx.y, dx.z, dx.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int v = 4 * g + e;
+          const float tv = float(Q4 ? (Ch[v] << 3) + Cl[v] : Ch[v] * 128 + Cl[v]);
+          acc[v] = fmaf(dxv[e], Q4 ? dw * tv - dm * Mn[v] : dw * tv, acc[v]);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  // the waves' sums, each in its own stage: [16 values][64 lanes]; wave w adds up values
+  // w, w + KW, ... in wave order
+  float* red = reinterpret_cast<float*>(&T);
+#pragma unroll
+  for (int v = 0; v < 16; v++) red[v * 64 + lane] = acc[v];
+  __syncthreads();
+  const int n = 32 * tn + lr;
+#pragma unroll
+  for (int j = 0; j < 16 / KW; j++) {
+    const int v = wv + KW * j;
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < KW; w++) sum += reinterpret_cast<const float*>(&S[w])[v * 64 + lane];
+    const int m = m0 + 8 * (v >> 2) + 4 * lh + (v & 3);
+    if (m < M && n < N) y[int64_t(m) * N + n] = sum;
+  }
+}
+
 int launch_gemm_layout(int quant, const void* w, int64_t n_in, int64_t n_out, void* dst, hipStream_t s) {
   if (!is_q4k(quant) && !is_q6k(quant))
     return fail(JERO_ERR_CAPABILITY_MISMATCH, "gemm layout: weights must be Q4_K, Q4_K_R, Q6_K or Q6_K_R");
@@ -827,11 +1006,33 @@ int launch_gemm_layout(int quant, const void* w, int64_t n_in, int64_t n_out, vo
 }
 
 int launch_gemm_laid(int laid, const void* w, int64_t n_in, int64_t n_out, const void* xq, int64_t m, float* y,
-                     hipStream_t s, float* y2, bool* split_out) {
+                     hipStream_t s, float* y2, bool* split_out, bool beside) {
   const int nb = int(n_in / 256);
   const int64_t tiles = ((m + kGpBM - 1) / kGpBM) * ((n_out + kGpBN - 1) / kGpBN);
+  // Few (32-token, 32-row) tiles: K split over the waves, eight of them while the tiles leave CUs
+  // empty.  In us, 64 x 128 tiles in K halves against this (tiles in brackets): Q4_K_G 4096 -> 1024 37
+  // tokens (64) 17.8 and 7.7, 512 (512) 21.2 and 13.3; 4096 -> 4096 128 (512) 20.7 and 15.0, 192 (768)
+  // 23.2 and 20.8, 256 (1024) 25.6 and 25.0; 4096 -> 14336 32 (448) 21.0 and 15.6, 64 (896) 24.7 and
+  // 25.3; 12288 -> 1024 512 (512) 43.4 and 29.7, 768 (768) 45.8 and 48.8; Q6_K_P 12288 -> 4096 37
+  // (256) 59.8 and 29.3, 128 (512) 59.9 and 46.7, 192 (768) 60.6 and 61.3.  Beside another launch
+  // that fills most of the GPU the fewer workgroups of the tiles hide better (attn_v of 512 tokens:
+  // a 1.46 ms prefill took 1.2 % longer).
+  const int64_t cus = device_info().cus;
+  const int64_t kw_tiles = ((m + 31) / 32) * ((n_out + 31) / 32);
+  if (kw_tiles <= (m <= 192 ? 3 : 2) * cus && !(beside && m > 128)) {
+    if (split_out) *split_out = false;
+    const bool wide = kw_tiles <= cus;
+    const dim3 grid{unsigned(kw_tiles)}, block(wide ? 512 : 256);
+    const uint8_t* xb = static_cast<const uint8_t*>(xq);
+    const uint8_t* wb = static_cast<const uint8_t*>(w);
+    const int64_t xrb = row_bytes(JERO_Q8_K, n_in);
+    auto* const kernel = laid == JERO_Q4_K_G ? (wide ? gemm_laid_kw_kernel<true, 8> : gemm_laid_kw_kernel<true, 4>)
+                                             : (wide ? gemm_laid_kw_kernel<false, 8> : gemm_laid_kw_kernel<false, 4>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y);
+    return check_launch("gemm (few tokens)");
+  }
   // two workgroups per CU: a grid that fills at most half of that splits K in two
-  const bool split = nb >= 2 && tiles <= device_info().cus;
+  const bool split = nb >= 2 && tiles <= cus;
   if (split_out) *split_out = split && y2;
   const uint8_t* xb = static_cast<const uint8_t*>(xq);
   const uint8_t* wb = static_cast<const uint8_t*>(w);
@@ -914,15 +1115,20 @@ using namespace jero;
 
 namespace jero {
 
+// Rows from which a Q4_K tensor whose rows are not a multiple of the tile runs the MFMA kernel rather
+// than one GEMV per row (4096 -> 1056: 8 rows 19 us as GEMVs and 27 here, 16 rows 37 and 27, 256 rows
+// 554 and 28; 2048 -> 5024: 8 rows 24 and 17).
+constexpr int64_t kRaggedMinRows = 16;
+
 int launch_gemm(int quant, const void* w_dev, int64_t n_in, int64_t n_out, const void* xq_dev, int64_t m, float* y_dev,
-                hipStream_t s, const void* laid, float* y2, bool* split_out) {
+                hipStream_t s, const void* laid, float* y2, bool* split_out, bool beside) {
   if (split_out) *split_out = false;
   const int act = act_format(quant);
   const int64_t xrb = row_bytes(act, n_in);
   if (quant == JERO_Q4_K_G || quant == JERO_Q6_K_P) return launch_gemm_laid(quant, w_dev, n_in, n_out, xq_dev, m, y_dev, s);
   if ((is_q4k(quant) || is_q6k(quant)) && laid)
     return launch_gemm_laid(is_q4k(quant) ? JERO_Q4_K_G : JERO_Q6_K_P, laid, n_in, n_out, xq_dev, m, y_dev, s, y2,
-                            split_out);
+                            split_out, beside);
   if (is_q6k(quant) && m >= kLaidMinRows) {  // the Q6_K_P planes built into the library workspace for this call
     void* ws = nullptr;
     int rc = workspace(gemm_layout_bytes(quant, n_in, n_out), &ws);
@@ -930,7 +1136,7 @@ int launch_gemm(int quant, const void* w_dev, int64_t n_in, int64_t n_out, const
     if (rc) return rc;
     return launch_gemm_laid(JERO_Q6_K_P, ws, n_in, n_out, xq_dev, m, y_dev, s);
   }
-  if ((quant == JERO_Q4_K || quant == JERO_Q4_K_R) && n_out % kGemmBN == 0) {
+  if ((quant == JERO_Q4_K || quant == JERO_Q4_K_R) && (n_out % kGemmBN == 0 || m >= kRaggedMinRows)) {
     const int tiles = gemm_tiles(m, n_out);
     const int nb = int(n_in / 256);
     // at most half the CUs busy (one 115 KB workgroup per CU): two workgroups per tile, one per

@@ -1318,7 +1318,8 @@ extern "C" int jero_hip_model_prefill(jero_model* m, const int32_t* tokens, int6
         vp = b.QKV + n * w1, vs = KV;
         const void* laid_v = nullptr;
         if ((rc = laid_of(m, l.wv, s, &laid_v)) || (rc = fork_side(m, s)) ||
-            (rc = launch_gemm(l.wv.quant, l.wv.dev, H, l.wv.n_out, b.XQ, n, vp, m->side, laid_v, b.T2, &vsplit)))
+            (rc = launch_gemm(l.wv.quant, l.wv.dev, H, l.wv.n_out, b.XQ, n, vp, m->side, laid_v, b.T2, &vsplit,
+                              true)))
           return rc;
       }
       if ((rc = project(l.qkv, b.XN, H, b.QKV, TraceLayout::kQ8Attn))) return rc;
