@@ -22,9 +22,11 @@
 //   down  : requant, saturating add into x
 // then the head (RMSNorm of the last row, int32 logits).  In evaluate, the next step's first launch
 // samples the greedy token from those logits and embeds it in every workgroup's prologue (one
-// workgroup also stores the token and the row): the decode loop never waits for the host.  Up to kMvRows rows the projections run on the matvec kernel below
-// (one weight row per wave, the token rows in LDS); longer prompts run the int8 MFMA GEMM of
-// gemm.hip with the same fused epilogues, after a row RMSNorm kernel.
+// workgroup also stores the token and the row): the decode loop never waits for the host.  Up to
+// kDecPos positions all of evaluate's decode steps run in one launch instead (fwd_decode_kernel).  Up
+// to kMvRows rows the projections run on the matvec kernel below (one weight row per wave, the token
+// rows in LDS); longer prompts run the int8 MFMA GEMM of gemm.hip with the same fused epilogues,
+// after a row RMSNorm kernel.
 #include <algorithm>
 #include <string>
 #include <vector>
@@ -92,23 +94,22 @@ __device__ __forceinline__ uint32_t floor_sqrt_u24(uint32_t v) {
 
 // ForwardExec::rmsnorm (src/forward.rs:672-699) of one 512-byte row held by a wave, 8 bytes per
 // lane: rms = max(isqrt(sum v^2 / 512), 1), y = clamp(v * 48 / rms, -127, 127) (division
-// truncating toward zero).  |v * 48| <= 6144 and rms <= 128, so the quotient is the high word of
-// |v * 48| * ceil(2^32 / rms), exact (division by an invariant integer, Granlund & Montgomery
-// 1994: the error term stays below |v * 48| / 2^32 < 1 / rms).
+// truncating toward zero).  The quotient is taken in f32, exactly: (|v * 48| + 1/2) / rms lies at
+// least 1 / (2 rms) from every integer, and the roundings of it (1 / rms, 48 / rms and the fma) move
+// it by less than 2^-22 of itself, which is below 6145 * 2^-22 / rms.
 __device__ __forceinline__ void rmsnorm_lane(uint32_t (&v)[2]) {
   int ss = dot4(v[0], v[0], dot4(v[1], v[1], 0));
   ss = __builtin_amdgcn_readlane(wave_sum_last_i(ss), 63);
   const uint32_t rms = max(floor_sqrt_u24(uint32_t(ss) / kFwdDim), 1u);
-  const uint32_t mul = rms == 1 ? 0u : 0xFFFFFFFFu / rms + 1u;  // ceil(2^32 / rms) for rms > 1
+  const float inv = 1.0f / float(rms), m48 = 48.0f * inv;
 #pragma unroll
   for (int d = 0; d < 2; d++) {
     uint32_t o = 0;
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-      const int x = int(int8_t(byte_of(v[d], b))) * 48;
-      const uint32_t ax = uint32_t(x < 0 ? -x : x);
-      const int q = int(rms == 1 ? ax : __umulhi(ax, mul));
-      o |= uint32_t(uint8_t(clamp_i8(x < 0 ? -q : q, -127))) << (8 * b);
+      const float x = float(int(int8_t(byte_of(v[d], b))));
+      const int q = int(fmaf(x, m48, copysignf(0.5f * inv, x)));
+      o |= uint32_t(uint8_t(int8_t(min(max(q, -127), 127)))) << (8 * b);
     }
     v[d] = o;
   }
@@ -393,6 +394,334 @@ __global__ void __launch_bounds__(256) fwd_fill_kernel(uint64_t seed, int64_t va
     w[i] = i < valid ? int8_t(small_of(seed, uint64_t(i))) : int8_t(0);
 }
 
+// ---- evaluate's decode steps in one launch.
+// A step is 17 dependent products whose 8.5 MB of weights lie in the L2s: as 17 launches it took
+// 50 us, nearly all of it launch boundaries (about 2.5 us each).  Here kDecWgs workgroups run every
+// step of an evaluate.  Each of the 128 waves owns four consecutive rows of every 512-row matrix
+// (eight of up, one 16-lane group per row), and each phase's output goes from wave to wave as 8-byte
+// words in device memory: a payload (four int8 rows, or one logit) and the phase's tag, written and
+// read by relaxed device-scope atomics.  A word carries its own arrival, so no fence, counter or
+// barrier orders anything across workgroups: a reader loads the words until all carry its tag.  A
+// buffer is rewritten only a layer later, by waves that have read words of every wave that read it:
+// each wave publishes a phase after it has read the phase before.  Every word is written to
+// kDecCopies places, and a workgroup reads the copy of its index: with one copy the readers of its
+// few lines queued up (46 us a step against 41; 32 copies: 44).  The weights of the next phase are
+// loaded before the wait for its input, the K / V rows before the projections'.  Attention runs in
+// every workgroup (as in the launches): the positions of this evaluate come from the workgroup's own
+// copy of the K / V rows, which only it writes, those of the prompt from the caches, the newest row
+// from the exchange.  A step takes 36 us; what bounds it is the 17 exchanges (a store to memory and a
+// read of it, about 1.5 us).
+// All workgroups have to be resident: the launch is cooperative.  A wave that waits in vain for
+// kDecSpins reads stops publishing, so every wait ends, and token 2^32 - 1 reports it.
+constexpr int kDecWgs = 32, kDecWaves = kDecWgs * kMvWaves;
+constexpr int kDecWords = kFwdDim / 4;     // words of a model row
+constexpr int kDecHeadRows = 4096;         // head rows (exchange words) at most
+constexpr int kDecPos = int(kAttInMax);    // positions at most
+constexpr int kDecTags = 4 * kFwdLayers + 1;  // exchanges per step
+constexpr int kDecSpins = 1 << 22;
+constexpr int kDecCopies = 8;  // of every word
+static_assert(kDecWaves == kDecWords, "a wave owns one word of a model row");
+
+struct DecXch {
+  uint64_t qkv[3 * kDecWords], x1[kDecWords], up[2 * kDecWords], x2[kDecWords], logits[kDecHeadRows];
+};
+
+struct DecArgs {
+  const int8_t* w[kFwdLayers][kFwdMats];
+  const int8_t* head;
+  int8_t *kc[kFwdLayers], *vc[kFwdLayers];
+  int8_t* own;  // [kDecWgs][kFwdLayers][2][rows][512]
+  int own_rows;
+  DecXch* x;  // [kDecCopies]
+  const int32_t* logits0;  // the prompt's logits
+  uint32_t* toks;
+  int n, max_tokens, vocab, head_rows;
+  uint32_t tag;
+  uint64_t seed;
+};
+
+struct DecWait {
+  int left = kDecSpins;
+  __device__ __forceinline__ bool dead() const { return left <= 0; }
+};
+
+// v[j] = the payload of word lane + STRIDE j (clamped to the last of n), once all carry the tag.
+template <int NW, int STRIDE = 64>
+__device__ __forceinline__ void dec_read(const uint64_t* __restrict__ words, int n, uint32_t tag, uint32_t (&v)[NW],
+                                         DecWait& W) {
+  const int lane = threadIdx.x & 63;
+  while (W.left > 0) {
+    uint64_t r[NW];
+#pragma unroll
+    for (int j = 0; j < NW; j++)
+      r[j] = __hip_atomic_load(words + min(lane + STRIDE * j, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < NW; j++) {
+      ok = ok && uint32_t(r[j] >> 32) == tag;
+      v[j] = uint32_t(r[j]);
+    }
+    if (__all(ok)) return;
+    W.left--;
+  }
+}
+
+// The word (of the first copy) into every copy; called by whole waves.
+__device__ __forceinline__ void dec_write(uint64_t* word, uint32_t tag, uint32_t v, const DecWait& W) {
+  const int c = threadIdx.x & 63;
+  if (c < kDecCopies && !W.dead())
+    __hip_atomic_store(word + c * (sizeof(DecXch) / sizeof(uint64_t)), (uint64_t(tag) << 32) | v, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The bytes of the four 16-lane groups (each uniform in its group) as one word.
+__device__ __forceinline__ uint32_t dec_pack(int v) {
+  return (uint32_t(__builtin_amdgcn_readlane(v, 0)) & 0xFFu) | (uint32_t(__builtin_amdgcn_readlane(v, 16)) & 0xFFu) << 8 |
+         (uint32_t(__builtin_amdgcn_readlane(v, 32)) & 0xFFu) << 16 | uint32_t(__builtin_amdgcn_readlane(v, 48)) << 24;
+}
+
+// D dwords (a lane's 1/16) of one row.
+template <int D>
+struct DecRow {
+  u32x4 v[D / 4];
+};
+template <int D>
+__device__ __forceinline__ void dec_load(DecRow<D>& R, const int8_t* __restrict__ w, int64_t row) {
+  const uint8_t* p = reinterpret_cast<const uint8_t*>(w) + (row * 16 + (threadIdx.x & 15)) * (4 * D);
+#pragma unroll
+  for (int i = 0; i < D / 4; i++) R.v[i] = ld4(p + 16 * i);
+}
+// The row's sum over its 16 lanes, in each of them; x: the lane's slice of the input row.
+template <int D>
+__device__ __forceinline__ int dec_dot(const DecRow<D>& R, const DecRow<D>& x) {
+  int acc = 0;
+#pragma unroll
+  for (int i = 0; i < D / 4; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc = dot4(R.v[i][e], x.v[i][e], acc);
+  return row_sum_i(acc);
+}
+__device__ __forceinline__ int dec_requant(int acc, int shift) {
+  return clamp_i8(int(int32_t(uint32_t(acc) + (uint32_t(1) << (shift - 1))) >> shift), -127);
+}
+
+struct DecSmem {
+  uint32_t in[kMvWaves][2 * kDecWords];  // a wave's input row
+  uint32_t qkv[3 * kDecWords];           // the newest q, k and v rows
+  int8_t att[kFwdDim];
+  AttSmem att_s;
+};
+
+// The lane's slice of the wave's input row (words lane + 64 j in v).
+template <int NW>
+__device__ __forceinline__ void dec_slice(uint32_t* in, const uint32_t (&v)[NW], DecRow<4 * NW>& x) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int j = 0; j < NW; j++) in[lane + 64 * j] = v[j];
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < NW; i++) x.v[i] = *reinterpret_cast<const u32x4*>(&in[(lane & 15) * 4 * NW + 4 * i]);
+  __builtin_amdgcn_wave_barrier();
+}
+
+// K and V rows of the 64 positions from b0 (attend_row's shares): position j < n from the caches,
+// j < pos from the workgroup's own rows; later ones repeat the last.
+__device__ __forceinline__ void dec_load_kv(const DecArgs& a, int l, const int8_t* own_k, const int8_t* own_v, int b0,
+                                            int pos, u32x4 (&k)[4][2], u32x4 (&v)[8]) {
+  const int t = threadIdx.x, kj = t >> 4, sub = t & 15, grp = t >> 5, c16 = (t & 31) * 16;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    if (b0 + 16 * u >= pos) break;
+    const int j = min(b0 + kj + 16 * u, pos - 1);
+    const uint8_t* r = reinterpret_cast<const uint8_t*>(j < a.n ? a.kc[l] : own_k) + int64_t(j) * kFwdDim + sub * 32;
+    k[u][0] = ld4(r), k[u][1] = ld4(r + 16);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    if (b0 + 8 * i >= pos) break;
+    const int j = min(b0 + grp + 8 * i, pos - 1);
+    v[i] = ld4(reinterpret_cast<const uint8_t*>(j < a.n ? a.vc[l] : own_v) + int64_t(j) * kFwdDim + c16);
+  }
+}
+
+// attend_row over positions 0..pos, the last in S.qkv, the first 64 of the others in k and v.
+__device__ __forceinline__ void dec_attend(const DecArgs& a, int l, const int8_t* own_k, const int8_t* own_v, int pos,
+                                           u32x4 (&k)[4][2], u32x4 (&v)[8], DecSmem& S) {
+  const int t = threadIdx.x, kj = t >> 4, sub = t & 15, grp = t >> 5, c16 = (t & 31) * 16;
+  const u32x4 q0 = *reinterpret_cast<const u32x4*>(&S.qkv[sub * 8]);
+  const u32x4 q1 = *reinterpret_cast<const u32x4*>(&S.qkv[sub * 8 + 4]);
+  int acc[16] = {}, tw = 0, buf = 0;
+  for (int b0 = 0; b0 <= pos; b0 += 64) {
+    if (b0) dec_load_kv(a, l, own_k, own_v, b0, pos, k, v);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (b0 + 16 * u > pos) break;
+      if (b0 + kj + 16 * u == pos) {
+        k[u][0] = *reinterpret_cast<const u32x4*>(&S.qkv[kDecWords + sub * 8]);
+        k[u][1] = *reinterpret_cast<const u32x4*>(&S.qkv[kDecWords + sub * 8 + 4]);
+      }
+      int sc = 0;
+#pragma unroll
+      for (int d = 0; d < 4; d++) sc = dot4(q0[d], k[u][0][d], dot4(q1[d], k[u][1][d], sc));
+      const int sh = row_sum_i(sc) >> 10;
+      if (sub == 0) S.att_s.wts[buf][kj + 16 * u] = uint8_t((sh < 0 ? 0 : sh > 127 ? 127 : sh) + 1);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (b0 + 8 * i > pos) break;
+      const int j = grp + 8 * i;
+      if (b0 + j == pos) v[i] = *reinterpret_cast<const u32x4*>(&S.qkv[2 * kDecWords + (t & 31) * 4]);
+      const int w = b0 + j <= pos ? int(S.att_s.wts[buf][j]) : 0;
+#pragma unroll
+      for (int b = 0; b < 16; b++) acc[b] += w * int(int8_t(byte_of(v[i][b >> 2], b & 3)));
+      tw += w;
+    }
+    buf ^= 1;
+  }
+#pragma unroll
+  for (int b = 0; b < 16; b += 4)
+    *reinterpret_cast<int4*>(&S.att_s.part[grp][c16 + b]) = int4{acc[b], acc[b + 1], acc[b + 2], acc[b + 3]};
+  if ((t & 31) == 0) S.att_s.tw[grp] = tw;
+  __syncthreads();
+  int s0 = 0, s1 = 0, st = 0;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int2 pr = *reinterpret_cast<const int2*>(&S.att_s.part[i][2 * t]);
+    s0 += pr.x, s1 += pr.y, st += S.att_s.tw[i];
+  }
+  S.att[2 * t] = int8_t(s0 / st);  // kDecPos * 128 * 127 fits 32 bits
+  S.att[2 * t + 1] = int8_t(s1 / st);
+  __syncthreads();
+}
+
+__global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
+  __shared__ __attribute__((aligned(16))) DecSmem S;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, g = lane >> 4;
+  const int gw = blockIdx.x * kMvWaves + wv;  // this wave's word of a model row
+  const int64_t r4 = 4 * gw + g;              // this lane group's row of a 512-row matrix
+  const int64_t own_row = int64_t(a.own_rows) * kFwdDim;
+  int8_t* const own = a.own + int64_t(blockIdx.x) * (2 * kFwdLayers) * own_row;
+  DecXch& X0 = a.x[0];
+  DecXch& X = a.x[blockIdx.x % kDecCopies];
+  DecWait W;
+  uint32_t tag = a.tag;
+  for (int i = 1;; i++) {
+    DecRow<8> wq[3];
+#pragma unroll
+    for (int p = 0; p < 3; p++) dec_load(wq[p], a.w[0][p], r4);
+    // the greedy token of the last logits: their first maximum (ForwardModel::sample)
+    const int nv = a.vocab > 1 ? a.vocab : 1;
+    int bv = INT32_MIN, bi = INT32_MAX;
+    for (int c0 = 0; c0 < nv; c0 += 256) {
+      uint32_t lg[4] = {0u, 0u, 0u, 0u};
+      if (i == 1) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) lg[j] = uint32_t(a.logits0[c0 + min(lane + 64 * j, nv - c0 - 1)]);
+      } else {
+        dec_read(X.logits + c0, nv - c0, tag, lg, W);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (c0 + lane + 64 * j < nv && (bi == INT32_MAX || int(lg[j]) > bv)) bv = int(lg[j]), bi = c0 + lane + 64 * j;
+    }
+    const int vmax = wave_max_i(bi == INT32_MAX ? INT32_MIN : bv);
+    const uint32_t tok = uint32_t(wave_min_i(bi != INT32_MAX && bv == vmax ? bi : INT32_MAX));
+    if (gw == 0 && lane == 0) a.toks[i - 1] = W.dead() ? ~0u : tok;
+    if (i == a.max_tokens) break;
+    const int pos = a.n + i - 1;
+    // its embedding: words lane and lane + 64 of the row
+    uint32_t v[2] = {0u, 0u};
+    const uint64_t sd = a.seed ^ (uint64_t(tok) * 0x9E3779B9ull);
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      v[e >> 2] |= uint32_t(uint8_t(int8_t(small_of(sd, uint64_t((e >> 2) * 256 + lane * 4 + (e & 3))) * 8))) << (8 * (e & 3));
+    uint32_t mine = uint32_t(__builtin_amdgcn_readlane(int(gw < 64 ? v[0] : v[1]), gw & 63));  // the wave's rows of x
+    DecRow<8> x;
+    for (int l = 0; l < kFwdLayers; l++) {
+      int8_t* const own_k = own + (2 * l) * own_row;
+      int8_t* const own_v = own_k + own_row;
+      u32x4 k[4][2], vv[8];
+      if (l) {
+#pragma unroll
+        for (int p = 0; p < 3; p++) dec_load(wq[p], a.w[l][p], r4);
+      }
+      dec_load_kv(a, l, own_k, own_v, 0, pos, k, vv);
+      if (l) {
+        dec_read(X.x2, kDecWords, tag, v, W);
+      }
+      rmsnorm_lane(v);
+      dec_slice(S.in[wv], v, x);
+      tag++;
+#pragma unroll
+      for (int p = 0; p < 3; p++) {
+        const uint32_t word = dec_pack(dec_requant(dec_dot(wq[p], x), 6));
+        dec_write(&X0.qkv[p * kDecWords + gw], tag, word, W);
+        if (lane == 0 && p) {
+          reinterpret_cast<uint32_t*>((p == 1 ? a.kc : a.vc)[l] + int64_t(pos) * kFwdDim)[gw] = word;
+        }
+      }
+      DecRow<8> wo, wu[2];
+      dec_load(wo, a.w[l][3], r4);
+      {  // word t of q | k | v, and word 256 + t of the first two waves
+        uint32_t one[1] = {0u}, two[2] = {0u, 0u};
+        if (wv < 2) {
+          dec_read<2, 256>(X.qkv + 64 * wv, 3 * kDecWords, tag, two, W);
+          S.qkv[t] = two[0];
+          S.qkv[256 + t] = two[1];
+          reinterpret_cast<uint32_t*>(own_v + int64_t(pos) * kFwdDim)[t] = two[1];
+        } else {
+          dec_read(X.qkv + 64 * wv, 64, tag, one, W);
+          S.qkv[t] = one[0];
+          reinterpret_cast<uint32_t*>(own_k + int64_t(pos) * kFwdDim)[t - kDecWords] = one[0];
+        }
+      }
+      __syncthreads();
+      dec_attend(a, l, own_k, own_v, pos, k, vv, S);
+#pragma unroll
+      for (int e = 0; e < 2; e++) x.v[e] = *reinterpret_cast<const u32x4*>(&S.att[(lane & 15) * 32 + 16 * e]);
+      tag++;
+      int y = clamp_i8(int(int8_t(byte_of(mine, g))) + dec_requant(dec_dot(wo, x), 6), -128);
+      mine = dec_pack(y);
+      dec_write(&X0.x1[gw], tag, mine, W);
+#pragma unroll
+      for (int p = 0; p < 2; p++) dec_load(wu[p], a.w[l][4], 8 * gw + 4 * p + g);
+      dec_read(X.x1, kDecWords, tag, v, W);
+      rmsnorm_lane(v);
+      dec_slice(S.in[wv], v, x);
+      tag++;
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        const uint32_t word = dec_pack(max(dec_requant(dec_dot(wu[p], x), 6), 0));
+        dec_write(&X0.up[2 * gw + p], tag, word, W);
+      }
+      DecRow<16> wd, xu;
+      dec_load(wd, a.w[l][5], r4);
+      uint32_t u4[4] = {0u, 0u, 0u, 0u};
+      dec_read(X.up, 2 * kDecWords, tag, u4, W);
+      dec_slice(S.in[wv], u4, xu);
+      tag++;
+      y = clamp_i8(int(int8_t(byte_of(mine, g))) + dec_requant(dec_dot(wd, xu), 7), -128);
+      mine = dec_pack(y);
+      dec_write(&X0.x2[gw], tag, mine, W);
+    }
+    DecRow<8> wh;
+    dec_load(wh, a.head, min(r4, int64_t(a.head_rows - 1)));
+    dec_read(X.x2, kDecWords, tag, v, W);
+    rmsnorm_lane(v);
+    dec_slice(S.in[wv], v, x);
+    tag++;
+    for (int64_t r = r4; r - g < a.head_rows; r += kFwdDim) {
+      if (r >= kFwdDim) dec_load(wh, a.head, min(r, int64_t(a.head_rows - 1)));
+      const int acc = dec_dot(wh, x);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (r - g + q < a.head_rows)
+          dec_write(&X0.logits[r - g + q], tag, uint32_t(__builtin_amdgcn_readlane(acc, 16 * q)), W);
+    }
+  }
+}
+
 }  // namespace jero
 
 using namespace jero;
@@ -413,6 +742,11 @@ struct jero_forward_model {
   hipStream_t gs = nullptr;
   hipGraphExec_t graph = nullptr;
   int64_t graph_n = -1, graph_max = -1;
+  // evaluate's decode steps in one launch (null: the graph): the exchange and the workgroups' own
+  // K / V rows; xtag counts the exchanges made so far
+  DecXch* xch = nullptr;
+  int8_t* own = nullptr;
+  uint32_t xtag = 0;
 };
 
 namespace {
@@ -563,6 +897,30 @@ int capture_decode(jero_forward_model* f, int64_t n, int64_t max_tokens) {
   return JERO_OK;
 }
 
+// evaluate's decode steps as one launch of fwd_decode_kernel on gs; false, with nothing launched,
+// where the graph takes them: no buffers, more positions or head rows than it is made for, or a
+// device that refuses the cooperative launch.
+bool launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens) {
+  if (!f->xch || max_tokens < 2 || n + max_tokens - 1 > kDecPos) return false;
+  DecArgs a{};
+  for (int l = 0; l < kFwdLayers; l++) {
+    for (int j = 0; j < kFwdMats; j++) a.w[l][j] = f->w[l][j];
+    a.kc[l] = f->kc[l], a.vc[l] = f->vc[l];
+  }
+  a.head = f->head, a.own = f->own, a.own_rows = int(std::min<int64_t>(f->cap, kDecPos)), a.x = f->xch;
+  a.logits0 = f->logits, a.toks = f->tokens;
+  a.n = int(n), a.max_tokens = int(max_tokens), a.vocab = int(f->vocab), a.head_rows = int(f->head_rows);
+  a.tag = f->xtag, a.seed = f->seed;
+  void* args[] = {&a};
+  if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fwd_decode_kernel), dim3(kDecWgs), dim3(kMvWaves * 64),
+                                 args, 0, f->gs) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  f->xtag += uint32_t(kDecTags * (max_tokens - 1));
+  return true;
+}
+
 int check_model(const jero_forward_model* f, const char* who) {
   if (!f) return fail(JERO_ERR_INVALID_ARGUMENT, std::string(who) + ": null model");
   int dev = -1;
@@ -608,6 +966,21 @@ extern "C" int jero_hip_forward_model_create(uint64_t seed, int64_t vocab, int64
   if (!rc && !(rc = fwd_alloc(f, size_t(f->head_rows) * kFwdDim, &p))) f->head = static_cast<int8_t*>(p);
   if (!rc && !(rc = fwd_alloc(f, size_t(f->head_rows) * sizeof(int32_t), &p))) f->logits = static_cast<int32_t*>(p);
   if (!rc && !(rc = fwd_alloc(f, cap * sizeof(uint32_t), &p))) f->tokens = static_cast<uint32_t*>(p);
+  // the one-launch decode's buffers (17 MB at most); without them evaluate replays a graph
+  const size_t own_rows = std::min<size_t>(cap, kDecPos);
+  if (!rc && f->head_rows <= kDecHeadRows) {
+    void *px = nullptr, *po = nullptr;
+    if (hipMalloc(&px, kDecCopies * sizeof(DecXch)) == hipSuccess &&
+        hipMalloc(&po, size_t(kDecWgs) * kFwdLayers * 2 * own_rows * kFwdDim) == hipSuccess &&
+        hipMemset(px, 0, kDecCopies * sizeof(DecXch)) == hipSuccess) {
+      f->owned.push_back(px), f->owned.push_back(po);
+      f->xch = static_cast<DecXch*>(px), f->own = static_cast<int8_t*>(po);
+    } else {
+      (void)hipGetLastError();
+      (void)hipFree(px);
+      (void)hipFree(po);
+    }
+  }
   // ForwardModel::new (src/forward.rs:879-903): layer l's matrices from splitmix(seed ^ (16 l + j)),
   // j = 1..6 for wq wk wv wo up down; the head from splitmix(seed ^ 0xFFFF), max(vocab, 1) rows.
   for (int l = 0; l < kFwdLayers && !rc; l++)
@@ -700,20 +1073,24 @@ extern "C" int jero_hip_forward_model_evaluate(jero_forward_model* f, const uint
   uint32_t* const toks = f->tokens;
   if (!rc) rc = forward_rows(f, n, 0, f->logits, nullptr, s);
   if (!rc) rc = check_hip(hipEventRecord(ev[1], s), "event");
-  // The decode steps run as one graph on the model's stream gs, after the prefill: the steps are
+  // The decode steps run on the model's stream gs, after the prefill: in one launch where that takes
+  // the shape, else as one graph: the steps are
   // the same launches for every evaluate of this (n, max_tokens), so they are captured once and
   // replayed (the host then enqueues one graph instead of ~17 launches per token).
   if (!rc && !f->gs) rc = check_hip(hipStreamCreateWithFlags(&f->gs, hipStreamNonBlocking), "forward stream");
   if (!rc) rc = check_hip(hipStreamWaitEvent(f->gs, ev[1], 0), "forward stream order");
-  if (!rc && max_tokens > 0 && (f->graph_n != n || f->graph_max != max_tokens || !f->graph))
+  const bool one = !rc && launch_decode(f, n, max_tokens);
+  if (!rc && !one && max_tokens > 0 && (f->graph_n != n || f->graph_max != max_tokens || !f->graph))
     rc = capture_decode(f, n, max_tokens);
-  if (!rc && max_tokens > 0) rc = check_hip(hipGraphLaunch(f->graph, f->gs), "forward decode graph");
+  if (!rc && !one && max_tokens > 0) rc = check_hip(hipGraphLaunch(f->graph, f->gs), "forward decode graph");
   if (!rc) rc = check_hip(hipEventRecord(ev[2], f->gs), "event");
   if (!rc && max_tokens > 0)
     rc = check_hip(hipMemcpyAsync(generated, toks, size_t(max_tokens) * sizeof(uint32_t), hipMemcpyDeviceToHost,
                                   f->gs),
                    "forward generated");
   if (!rc) rc = check_hip(hipStreamSynchronize(f->gs), "forward_model_evaluate");
+  if (!rc && one && generated[max_tokens - 1] == ~0u)
+    rc = fail(JERO_ERR_DEVICE, "forward_model_evaluate: the decode launch's workgroups did not reach each other");
   if (!rc && timing_ms) {
     rc = check_hip(hipEventElapsedTime(&timing_ms[0], ev[0], ev[1]), "event time");
     if (!rc) rc = check_hip(hipEventElapsedTime(&timing_ms[1], ev[1], ev[2]), "event time");
