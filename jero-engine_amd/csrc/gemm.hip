@@ -608,8 +608,10 @@ struct __attribute__((aligned(16))) GpStage {
   float dx[kGpBM];
 };
 
-// A thread's share of one activation block: a quarter of row t / 4 (64 q8 bytes) and, by quarter,
-// the row's d (quarter 0) or half of its bsums (quarters 1, 2).
+// A thread's share of one activation block: 16-byte piece t % 16 of rows 16 i + t / 16 (a wave's load
+// reads whole 256-byte runs of four rows; a quarter row per thread, 48 lines a load, took 1-3 %
+// longer: 512 x 4096 -> 6144 42.4 and 41.0 us) and, by t, the d of row t (t < 64) or half of the bsums of
+// row (t - 64) / 2 (t < 192).
 struct GpAct {
   u32x4 q[4];
   u32x4 tail;
@@ -617,28 +619,30 @@ struct GpAct {
 
 __device__ __forceinline__ void gp_load_act(GpAct& A, const uint8_t* __restrict__ xq, int64_t xrb, int m0, int M,
                                             int b) {
-  const int t = threadIdx.x, r = t >> 2, q = t & 3;
-  const uint8_t* xa = xq + int64_t(min(m0 + r, M - 1)) * xrb + int64_t(b) * 292;
+  const int t = threadIdx.x & (kGpThreads - 1);
+  const uint8_t* xb = xq + int64_t(b) * 292;
 #pragma unroll
-  for (int i = 0; i < 4; i++) A.q[i] = ld4(xa + 4 + 64 * q + 16 * i);
-  A.tail = ld4(xa + (q == 1 ? 260 : q == 2 ? 276 : 0));
+  for (int i = 0; i < 4; i++)
+    A.q[i] = ld4(xb + int64_t(min(m0 + 16 * i + (t >> 4), M - 1)) * xrb + 4 + 16 * (t & 15));
+  const bool bs = t >= 64 && t < 192;
+  A.tail = ld4(xb + int64_t(min(m0 + (bs ? (t - 64) >> 1 : t & 63), M - 1)) * xrb + (bs ? 260 + 16 * (t & 1) : 0));
 }
 
 template <bool BSUMS>
 __device__ __forceinline__ void gp_store_act(const GpAct& A, GpStage& S) {
-  const int t = threadIdx.x, r = t >> 2, q = t & 3;
+  const int t = threadIdx.x & (kGpThreads - 1);
 #pragma unroll
-  for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4*>(&S.a[r][64 * q + 16 * i]) = A.q[i];
-  if (q == 0) S.dx[r] = __uint_as_float(A.tail.x);
+  for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4*>(&S.a[16 * i + (t >> 4)][16 * (t & 15)]) = A.q[i];
+  if (t < 64) S.dx[t] = __uint_as_float(A.tail.x);
   if constexpr (BSUMS) {
-    if (q == 1 || q == 2) {
+    if (t >= 64 && t < 192) {
       const uint32_t bw[4] = {A.tail.x, A.tail.y, A.tail.z, A.tail.w};
       uint32_t hw[4];
 #pragma unroll
       for (int i = 0; i < 4; i++)
         hw[i] = uint32_t(__builtin_bit_cast(uint16_t, _Float16(float(int16_t(bw[i] & 0xFFFFu))))) |
                 (uint32_t(__builtin_bit_cast(uint16_t, _Float16(float(int16_t(bw[i] >> 16))))) << 16);
-      *reinterpret_cast<u32x4*>(&S.bs[r][8 * (q - 1)]) = u32x4{hw[0], hw[1], hw[2], hw[3]};
+      *reinterpret_cast<u32x4*>(&S.bs[(t - 64) >> 1][8 * (t & 1)]) = u32x4{hw[0], hw[1], hw[2], hw[3]};
     }
   }
 }
@@ -653,24 +657,26 @@ __device__ __forceinline__ void gp_store_act(const GpAct& A, GpStage& S) {
 // the block's integer sums are scaled into f32 accumulators.  Q4_K_G: per K pair the lane's
 // fragment is expanded to the planes a * q4, b * q4 of both sub-blocks and T = 8 Ta + Tb; the
 // mins term is one v_mfma_f32_32x32x16_f16 over the 16 bsums (|bsum| <= 2048 and m <= 63 are
-// exact in f16, sums below 2^24).  Q6_K_P: T = 128 Th + Tl.  Two workgroups share a CU.  SPLIT:
-// two workgroups per tile, one per half of the blocks, adding into the zeroed output (two
-// addends: the same sum in either order).
-template <bool Q4, bool SPLIT>
-__global__ void __launch_bounds__(kGpThreads, 2) gemm_laid_kernel(const uint8_t* __restrict__ xq, int64_t xrb,
-                                                                   const uint8_t* __restrict__ wg, int M, int N,
-                                                                   int nb, float* __restrict__ y,
-                                                                   float* __restrict__ y2) {
-  __shared__ GpStage S[2];
+// exact in f16, sums below 2^24).  Q6_K_P: T = 128 Th + Tl.  Two workgroups share a CU.  K in two
+// halves: kSplitGrid, two workgroups per tile that write y and y2 or, without y2, add into the zeroed
+// output (two addends: the same sum in either order); kSplitWg, one workgroup of eight waves, the
+// second four on the second half with stages of their own, their sums added through LDS at the end.
+enum { kSplitNone = 0, kSplitGrid = 1, kSplitWg = 2 };
+template <bool Q4, int SPLIT>
+__global__ void __launch_bounds__(kGpThreads * (SPLIT == kSplitWg ? 2 : 1), SPLIT == kSplitWg ? 1 : 2)
+    gemm_laid_kernel(const uint8_t* __restrict__ xq, int64_t xrb, const uint8_t* __restrict__ wg, int M, int N, int nb,
+                     float* __restrict__ y, float* __restrict__ y2) {
+  __shared__ GpStage SS[SPLIT == kSplitWg ? 2 : 1][2];
   constexpr int REC = Q4 ? kQ4gRec : kQ6pRec;
-  const int n_tiles_m = (M + kGpBM - 1) / kGpBM;
+  constexpr int WGS = SPLIT == kSplitGrid ? 2 : 1;  // workgroups per tile
   int tm, tn;
-  const int half = SPLIT ? int(blockIdx.x & 1) : 0;
-  gemm_tile_of(SPLIT ? int(blockIdx.x >> 1) : int(blockIdx.x), SPLIT ? int(gridDim.x >> 1) : int(gridDim.x),
-               n_tiles_m, tm, tn);
-  const int b0 = SPLIT ? half * ((nb + 1) / 2) : 0, b1 = SPLIT ? (half ? nb : (nb + 1) / 2) : nb;
+  gemm_tile_of(int(blockIdx.x) / WGS, int(gridDim.x) / WGS, (M + kGpBM - 1) / kGpBM, tm, tn);
+  const int half = SPLIT == kSplitWg ? int(threadIdx.x) / kGpThreads : SPLIT == kSplitGrid ? int(blockIdx.x & 1) : 0;
+  GpStage(&S)[2] = SS[SPLIT == kSplitWg ? half : 0];
+  const int nh = SPLIT ? (nb + 1) / 2 : nb;  // blocks of the first half; the second has as many or one less
+  const int b0 = half * nh, b1 = half ? nb : nh;
   const int m0 = tm * kGpBM;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
   const int lr = lane & 31, lh = lane >> 5;
   // this wave's record tile (clamped: a tile past N computes rows that are never stored)
   const int t32 = min(4 * tn + wv, (N + 31) / 32 - 1);
@@ -699,7 +705,11 @@ __global__ void __launch_bounds__(kGpThreads, 2) gemm_laid_kernel(const uint8_t*
   else dq = __uint_as_float(ld1(wr + int64_t(b0) * REC));
   gp_store_act<Q4>(A, S[0]);
   __syncthreads();
-  for (int b = b0; b < b1; b++) {
+  for (int b = b0; b < b0 + nh; b++) {
+    if (SPLIT && b >= b1) {  // an odd count of blocks: the second half has one less
+      if constexpr (SPLIT == kSplitWg) __syncthreads();
+      break;
+    }
     const GpStage& T = S[(b - b0) & 1];
     const int bn = min(b + 1, b1 - 1);  // the last block reloads itself: every load unconditional
     const int64_t on = int64_t(bn) * REC;
@@ -788,6 +798,18 @@ __global__ void __launch_bounds__(kGpThreads, 2) gemm_laid_kernel(const uint8_t*
     }
     __syncthreads();
   }
+  if constexpr (SPLIT == kSplitWg) {  // the second half's sums: [32 values][256 threads] over the stages
+    static_assert(sizeof(SS) >= 32 * kGpThreads * sizeof(float), "the sums fit the stages");
+    float* red = reinterpret_cast<float*>(&SS[0][0]) + (threadIdx.x & (kGpThreads - 1));
+    if (half) {
+#pragma unroll
+      for (int v = 0; v < 32; v++) red[v * kGpThreads] = acc[v >> 4][v & 15];
+    }
+    __syncthreads();
+    if (half) return;
+#pragma unroll
+    for (int v = 0; v < 32; v++) acc[v >> 4][v & 15] += red[v * kGpThreads];
+  }
   // store: for each v, the 32 lanes of a half-wave write 32 consecutive floats of one row
   const int n = 32 * (4 * tn + wv) + lr;
 #pragma unroll
@@ -796,7 +818,7 @@ __global__ void __launch_bounds__(kGpThreads, 2) gemm_laid_kernel(const uint8_t*
     for (int v = 0; v < 16; v++) {
       const int m = m0 + 32 * mt + 8 * (v >> 2) + 4 * lh + (v & 3);
       if (m < M && n < N) {
-        if constexpr (SPLIT) {
+        if constexpr (SPLIT == kSplitGrid) {
           if (y2) (half ? y2 : y)[int64_t(m) * N + n] = acc[mt][v];
           else atomicAdd(&y[int64_t(m) * N + n], acc[mt][v]);
         } else {
@@ -1031,29 +1053,29 @@ int launch_gemm_laid(int laid, const void* w, int64_t n_in, int64_t n_out, const
     hipLaunchKernelGGL(kernel, grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y);
     return check_launch("gemm (few tokens)");
   }
-  // two workgroups per CU: a grid that fills at most half of that splits K in two
-  const bool split = nb >= 2 && tiles <= cus;
-  if (split_out) *split_out = split && y2;
+  // A grid that fills at most half of two workgroups per CU splits K in two: over the grid for a
+  // caller that adds the halves itself, or where the tiles would leave half of the CUs empty; else
+  // within the workgroup, without the zeroed output and its atomics (512 tokens, us over the grid and
+  // within: Q4_K_G 4096 -> 4096 35.8 and 28.3, 1024 -> 4096 23.6 and 11.9, Q6_K_P 12288 -> 4096 91.0
+  // and 93.2; 256 tokens 12288 -> 4096, 128 tiles: 47.9 and 60.9).
+  const int split = nb < 2 || tiles > cus ? kSplitNone : y2 || 2 * tiles <= cus ? kSplitGrid : kSplitWg;
+  if (split_out) *split_out = split == kSplitGrid && y2;
   const uint8_t* xb = static_cast<const uint8_t*>(xq);
   const uint8_t* wb = static_cast<const uint8_t*>(w);
   const int64_t xrb = row_bytes(JERO_Q8_K, n_in);
-  const dim3 grid(unsigned(split ? 2 * tiles : tiles)), block(kGpThreads);
-  if (split) {
-    if (!y2) {  // both halves add into the zeroed output
-      hipLaunchKernelGGL(zero_f32_kernel, dim3(unsigned(std::min<int64_t>((m * n_out + 255) / 256, 4096))), dim3(256),
-                         0, s, y, m * n_out);
-      int rc = check_launch("gemm zero");
-      if (rc) return rc;
-    }
-    if (laid == JERO_Q4_K_G)
-      hipLaunchKernelGGL((gemm_laid_kernel<true, true>), grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y, y2);
-    else
-      hipLaunchKernelGGL((gemm_laid_kernel<false, true>), grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y, y2);
-  } else if (laid == JERO_Q4_K_G) {
-    hipLaunchKernelGGL((gemm_laid_kernel<true, false>), grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y, y2);
-  } else {
-    hipLaunchKernelGGL((gemm_laid_kernel<false, false>), grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y, y2);
+  if (split == kSplitGrid && !y2) {  // both halves add into the zeroed output
+    hipLaunchKernelGGL(zero_f32_kernel, dim3(unsigned(std::min<int64_t>((m * n_out + 255) / 256, 4096))), dim3(256), 0,
+                       s, y, m * n_out);
+    int rc = check_launch("gemm zero");
+    if (rc) return rc;
   }
+  const dim3 grid(unsigned(split == kSplitGrid ? 2 * tiles : tiles)), block(split == kSplitWg ? 2 * kGpThreads : kGpThreads);
+  const bool q4 = laid == JERO_Q4_K_G;
+  auto* const kernel =
+      split == kSplitGrid ? (q4 ? gemm_laid_kernel<true, kSplitGrid> : gemm_laid_kernel<false, kSplitGrid>)
+      : split == kSplitWg ? (q4 ? gemm_laid_kernel<true, kSplitWg> : gemm_laid_kernel<false, kSplitWg>)
+                          : (q4 ? gemm_laid_kernel<true, kSplitNone> : gemm_laid_kernel<false, kSplitNone>);
+  hipLaunchKernelGGL(kernel, grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y, y2);
   return check_launch(laid == JERO_Q4_K_G ? "gemm q4_k_g" : "gemm q6_k_p");
 }
 
