@@ -1299,17 +1299,38 @@ __global__ void __launch_bounds__(256, mfma_min_wgs(F, GU, PT)) moe_mfma_kernel(
   }
 }
 
+// y[t] (or resid[t] +=) = sum_j w[t, j] yd[inv[t, j]] in selection order, four outputs per thread and
+// per_token workgroups to a token, whose rows and weights are uniform loads: the rows' loads go out in
+// eights before the first sum.  One output per thread, each row's load waiting for its index, took
+// 16.5 us at 512 tokens x 8 x 2048 (33 MB read) against 8.6.  H % 4 == 0 (the experts' is H % 256).
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restrict__ yd, const float* __restrict__ w,
-                                                          const int32_t* __restrict__ inv, int T, int k, int H,
-                                                          float* __restrict__ y, int accumulate,
+                                                          const int32_t* __restrict__ inv, int k, int H,
+                                                          int per_token, float* __restrict__ y, int accumulate,
                                                           float* __restrict__ resid) {
-  const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= int64_t(T) * H) return;
-  const int t = int(idx / H), h = int(idx % H);
-  float acc = accumulate ? y[idx] : 0.f;
-  for (int j = 0; j < k; j++) acc += w[t * k + j] * yd[int64_t(inv[t * k + j]) * H + h];
-  if (resid) resid[idx] += acc;
-  else y[idx] = acc;
+  const int64_t t = int(blockIdx.x) / per_token;
+  const int h = 4 * (int(blockIdx.x) % per_token * 256 + int(threadIdx.x));
+  if (h >= H) return;
+  const float* wt = w + t * k;
+  const int32_t* it = inv + t * k;
+  float* out = (resid ? resid : y) + t * H + h;
+  f32x4_a4 acc = {0.f, 0.f, 0.f, 0.f};
+  const f32x4_a4 old = *reinterpret_cast<const f32x4_a4*>(resid || accumulate ? out : yd + h);
+  const bool seed = !resid && accumulate;
+  if (seed) acc = old;
+  for (int j0 = 0; j0 < k; j0 += 8) {
+    f32x4_a4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      v[u] = *reinterpret_cast<const f32x4_a4*>(yd + int64_t(it[min(j0 + u, k - 1)]) * H + h);
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (j0 + u < k)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] += wt[j0 + u] * v[u][e];
+  }
+  if (resid) acc += old;
+  *reinterpret_cast<f32x4_a4*>(out) = acc;
 }
 
 // ---------------------------------------------------------------- launch plumbing
@@ -1647,9 +1668,9 @@ int launch_moe(MoeArgs a, void* ws, hipStream_t s) {
   rc = check_launch("moe down");
   if (rc) return rc;
   }
-  const int64_t total = a.T * a.hidden;
-  hipLaunchKernelGGL(moe_combine_kernel, dim3(unsigned((total + 255) / 256)), dim3(256), 0, s, a.yd, a.sel_w, L.inv,
-                     int(a.T), a.top_k, int(a.hidden), a.y, int(a.accumulate), a.resid);
+  const int64_t per_token = (a.hidden + 1023) / 1024;
+  hipLaunchKernelGGL(moe_combine_kernel, dim3(unsigned(a.T * per_token)), dim3(256), 0, s, a.yd, a.sel_w, L.inv, a.top_k,
+                     int(a.hidden), int(per_token), a.y, int(a.accumulate), a.resid);
   return check_launch("moe combine");
 }
 

@@ -167,8 +167,8 @@ __global__ void __launch_bounds__(256) swiglu_rows_kernel(const float* __restric
 // given (the previous projection's residual, written back), XN[t] =
 // RMSNorm(X[t]) * w as rmsnorm_rows_kernel computes it (the same per-thread strided sums, so the
 // same bits), XN[t] also stored when XN is given, and Q[t] = the Q8_K blocks of XN[t] as
-// quant_q8k_kernel makes them (a wave per 256-block from LDS).  H a multiple of 256, at most
-// kFusedMaxH.
+// quant_q8k_kernel makes them (a wave per 256-block from LDS; none without Q).  H a multiple of 256,
+// at most kFusedMaxH.
 constexpr int kFusedMaxH = 8192;
 __global__ void __launch_bounds__(256) add_rmsnorm_q8k_rows_kernel(float* __restrict__ X, const float* __restrict__ D,
                                                                    const float* __restrict__ D2, int64_t H,
@@ -223,6 +223,7 @@ __global__ void __launch_bounds__(256) add_rmsnorm_q8k_rows_kernel(float* __rest
     }
   }
   __syncthreads();
+  if (!Q) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   uint8_t* q = Q + int64_t(blockIdx.x) * (H / 256) * 292;
   for (int64_t j = wv; j < H / 256; j += 4) {
@@ -279,6 +280,7 @@ __global__ void __launch_bounds__(256) add_rmsnorm_q8k_rows_fixed_kernel(float* 
     if (y) y[i] = u;
   }
   __syncthreads();
+  if (!Q) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   uint8_t* q = Q + int64_t(blockIdx.x) * PER * 292;
   for (int j = wv; j < PER; j += 4) {
@@ -320,9 +322,10 @@ __global__ void __launch_bounds__(256) swiglu_q8k_rows_kernel(const float* __res
 }
 
 // x[i] += d[i] (the residual of Wo and down).
-__global__ void __launch_bounds__(256) add_rows_kernel(float* __restrict__ x, const float* __restrict__ d, int64_t n) {
+__global__ void __launch_bounds__(256) add_rows_kernel(float* __restrict__ x, const float* __restrict__ d,
+                                                       const float* __restrict__ d2, int64_t n) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) x[i] += d[i];
+  if (i < n) x[i] += d2 ? d[i] + d2[i] : d[i];
 }
 
 }  // namespace
@@ -390,8 +393,8 @@ int launch_swiglu_q8k_rows(const float* g, int64_t g_stride, const float* u, int
   return check_launch("prefill swiglu + q8_k");
 }
 
-int launch_add_rows(float* x, const float* d, int64_t count, hipStream_t s) {
-  hipLaunchKernelGGL(add_rows_kernel, dim3(unsigned((count + 255) / 256)), dim3(256), 0, s, x, d, count);
+int launch_add_rows(float* x, const float* d, const float* d2, int64_t count, hipStream_t s) {
+  hipLaunchKernelGGL(add_rows_kernel, dim3(unsigned((count + 255) / 256)), dim3(256), 0, s, x, d, d2, count);
   return check_launch("prefill residual");
 }
 
