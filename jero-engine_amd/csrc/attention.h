@@ -40,6 +40,10 @@ struct AttnParams {
   // (part_o) and t * part_tok_ml (part_ml) floats on; all zero for one query
   int64_t q_stride, part_tok, part_tok_ml;
   int n_tok;  // queries of the batch (set by the launcher)
+  // set by the launcher for a single split: the partial kernel writes the output rows (query t's
+  // t * one_stride floats on) instead of partials
+  float* one_split;
+  int64_t one_stride;
 };
 
 int attn_splits(int active, int hd);
