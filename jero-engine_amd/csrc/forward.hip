@@ -422,7 +422,7 @@ constexpr int kDecSpins = 1 << 22;
 constexpr int kDecCopies = 8;  // of every word
 static_assert(kDecWaves == kDecWords, "a wave owns one word of a model row");
 
-struct DecXch {
+struct alignas(1024) DecXch {
   uint64_t qkv[3 * kDecWords], x1[kDecWords], up[2 * kDecWords], x2[kDecWords], logits[kDecHeadRows];
 };
 
@@ -969,16 +969,15 @@ extern "C" int jero_hip_forward_model_create(uint64_t seed, int64_t vocab, int64
   // the one-launch decode's buffers (17 MB at most); without them evaluate replays a graph
   const size_t own_rows = std::min<size_t>(cap, kDecPos);
   if (!rc && f->head_rows <= kDecHeadRows) {
-    void *px = nullptr, *po = nullptr;
-    if (hipMalloc(&px, kDecCopies * sizeof(DecXch)) == hipSuccess &&
-        hipMalloc(&po, size_t(kDecWgs) * kFwdLayers * 2 * own_rows * kFwdDim) == hipSuccess &&
-        hipMemset(px, 0, kDecCopies * sizeof(DecXch)) == hipSuccess) {
-      f->owned.push_back(px), f->owned.push_back(po);
-      f->xch = static_cast<DecXch*>(px), f->own = static_cast<int8_t*>(po);
+    void* px = nullptr;
+    const size_t words = kDecCopies * sizeof(DecXch);
+    if (hipMalloc(&px, words + size_t(kDecWgs) * kFwdLayers * 2 * own_rows * kFwdDim) == hipSuccess &&
+        hipMemset(px, 0, words) == hipSuccess) {
+      f->owned.push_back(px);
+      f->xch = static_cast<DecXch*>(px), f->own = static_cast<int8_t*>(px) + words;
     } else {
       (void)hipGetLastError();
       (void)hipFree(px);
-      (void)hipFree(po);
     }
   }
   // ForwardModel::new (src/forward.rs:879-903): layer l's matrices from splitmix(seed ^ (16 l + j)),

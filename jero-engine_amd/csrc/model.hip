@@ -1278,16 +1278,10 @@ extern "C" int jero_hip_model_prefill(jero_model* m, const int32_t* tokens, int6
           return r;
         return snap(fld(L, f_q8), b.XQ, size_t(xrb), size_t(xrb));
       }
-      // the same row step without the blocks: one pass over the rows instead of up to three launches
-      // (512 x 2048 with a split residual: two additions of 5 us and the norm)
-      const bool fused = H % 256 == 0 && H <= 8192;
-      if (fused) r = launch_add_rmsnorm_q8k_rows(b.X, pending, pending2, n, H, nw, eps, b.XN, nullptr, s);
-      else if (pending) r = launch_add_rows(b.X, pending, pending2, n * H, s);
-      if (r) return r;
+      if (pending && (r = launch_add_rows(b.X, pending, pending2, n * H, s))) return r;
       pending = pending2 = nullptr;
       have_fmt = -1;
-      if ((r = snap(fld(L, f_xin), b.X, 4 * H, 4 * H)) ||
-          (!fused && (r = launch_rmsnorm_rows(b.X, n, H, nw, eps, b.XN, s))))
+      if ((r = snap(fld(L, f_xin), b.X, 4 * H, 4 * H)) || (r = launch_rmsnorm_rows(b.X, n, H, nw, eps, b.XN, s)))
         return r;
       return snap(fld(L, f_xn), b.XN, 4 * H, 4 * H);
     };

@@ -165,10 +165,10 @@ __global__ void __launch_bounds__(256) swiglu_rows_kernel(const float* __restric
 // The fused row step before a projection over Q8_K activations, one workgroup per row t:
 // X[t] += D[t] (+ D2[t], added to D[t] first: the two K halves of a split projection) when D is
 // given (the previous projection's residual, written back), XN[t] =
-// RMSNorm(X[t]) * w as rmsnorm_rows_kernel computes it (the same per-thread strided sums, so the
-// same bits), XN[t] also stored when XN is given, and Q[t] = the Q8_K blocks of XN[t] as
-// quant_q8k_kernel makes them (a wave per 256-block from LDS; none without Q).  H a multiple of 256,
-// at most kFusedMaxH.
+// RMSNorm(X[t]) * w as rmsnorm_rows_kernel computes it (the same per-thread strided sums; in 11 of
+// 512 rows of 2048 the last bit differed), XN[t] also stored when XN is given, and Q[t] = the Q8_K blocks of XN[t] as
+// quant_q8k_kernel makes them (a wave per 256-block from LDS).  H a multiple of 256, at most
+// kFusedMaxH.
 constexpr int kFusedMaxH = 8192;
 __global__ void __launch_bounds__(256) add_rmsnorm_q8k_rows_kernel(float* __restrict__ X, const float* __restrict__ D,
                                                                    const float* __restrict__ D2, int64_t H,
@@ -223,7 +223,6 @@ __global__ void __launch_bounds__(256) add_rmsnorm_q8k_rows_kernel(float* __rest
     }
   }
   __syncthreads();
-  if (!Q) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   uint8_t* q = Q + int64_t(blockIdx.x) * (H / 256) * 292;
   for (int64_t j = wv; j < H / 256; j += 4) {
@@ -280,7 +279,6 @@ __global__ void __launch_bounds__(256) add_rmsnorm_q8k_rows_fixed_kernel(float* 
     if (y) y[i] = u;
   }
   __syncthreads();
-  if (!Q) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   uint8_t* q = Q + int64_t(blockIdx.x) * PER * 292;
   for (int j = wv; j < PER; j += 4) {
