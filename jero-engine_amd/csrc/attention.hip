@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(kAttnThreads) attn_partial_kernel(AttnParams p
       L += wt * s_l[w][h];
     }
     const int64_t row = int64_t(kh * group + h) * S + split;
-    if (p.one_split) {
+    if (!FUSED && p.one_split) {
       p.one_split[blockIdx.z * p.one_stride + row * HD + d] = o / L;
     } else {
       p.part_o[row * HD + d] = o;
@@ -699,7 +699,7 @@ __global__ void __launch_bounds__(kAttnThreads) attn_mfma_kernel(AttnParams p) {
       L += wt * s_l[w][h];
     }
     const int64_t row = int64_t(kh * group + h) * S + split;
-    if (p.one_split) {
+    if (!FUSED && p.one_split) {
       p.one_split[t0 * p.one_stride + row * HD + d] = ov / L;
     } else {
       p.part_o[row * HD + d] = ov;
@@ -1441,7 +1441,7 @@ static int attention_impl(AttnParams p, bool fused, int S, int T, float* out, in
   }
   // One split (up to 64 positions): the partial kernel divides its sums and writes the rows, without
   // the merge (one token, 32 heads of 128 over 8 KV heads, 1 / 64 positions: 7.5 / 7.8 us with it and
-  // 4.7 / 5.1 without).  An output that overlaps an input keeps the merge, which writes it after
+  // 4.7 / 5.1 without).  The decode step's rings have more than one split.  An output that overlaps an input keeps the merge, which writes it after
   // every workgroup has read.
   const int64_t rows = int64_t(T) * nq * p.hd * int64_t(sizeof(float));
   const int64_t kv = int64_t(p.active) * p.nkv * p.hd * (p.kv_dtype == JERO_KV_F16 ? 2 : 4);
@@ -1449,7 +1449,7 @@ static int attention_impl(AttnParams p, bool fused, int S, int T, float* out, in
     const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(x);
     return o < i + size_t(n) && i < o + size_t(rows);
   };
-  const bool direct = S == 1 && (fused || T > 1 || !(meets(p.q, rows) || meets(p.k, kv) || meets(p.v, kv)));
+  const bool direct = S == 1 && !fused && (T > 1 || !(meets(p.q, rows) || meets(p.k, kv) || meets(p.v, kv)));
   if (direct) p.one_split = out, p.one_stride = out_stride;
 #define JERO_ATTN_CASE(HDV)                                                                     \
   if (p.hd == HDV) {                                                                            \
