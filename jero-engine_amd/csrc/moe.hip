@@ -1299,10 +1299,10 @@ __global__ void __launch_bounds__(256, mfma_min_wgs(F, GU, PT)) moe_mfma_kernel(
   }
 }
 
-// y[t] (or resid[t] +=) = sum_j w[t, j] yd[inv[t, j]] in selection order, four outputs per thread and
-// per_token workgroups to a token, whose rows and weights are uniform loads: the rows' loads go out in
-// eights before the first sum.  One output per thread, each row's load waiting for its index, took
-// 16.5 us at 512 tokens x 8 x 2048 (33 MB read) against 8.6.  H % 4 == 0 (the experts' is H % 256).
+// r[t] = (accumulate ? y[t] : 0) + sum_j w[t, j] yd[inv[t, j]] in selection order, into y[t], or added
+// to resid[t] when given (y then only read).  Four outputs per thread and per_token workgroups to a
+// token, whose rows and weights are uniform loads: the rows' loads go out in eights before the first
+// sum.  One output per thread, each row's load waiting for its index, took 16.5 us at 512 tokens x 8 x 2048 (33 MB read) against 8.6.  H % 4 == 0 (the experts' is H % 256).
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restrict__ yd, const float* __restrict__ w,
                                                           const int32_t* __restrict__ inv, int k, int H,
@@ -1313,11 +1313,13 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restric
   if (h >= H) return;
   const float* wt = w + t * k;
   const int32_t* it = inv + t * k;
+  // the sum starts from y (accumulate) whether it then goes to y or onto resid: a shared expert's
+  // output lies in y when the decode step adds the layer to its residual
   float* out = (resid ? resid : y) + t * H + h;
+  const f32x4_a4 base = *reinterpret_cast<const f32x4_a4*>(accumulate ? y + t * H + h : yd + h);
+  const f32x4_a4 old = *reinterpret_cast<const f32x4_a4*>(resid ? out : yd + h);
   f32x4_a4 acc = {0.f, 0.f, 0.f, 0.f};
-  const f32x4_a4 old = *reinterpret_cast<const f32x4_a4*>(resid || accumulate ? out : yd + h);
-  const bool seed = !resid && accumulate;
-  if (seed) acc = old;
+  if (accumulate) acc = base;
   for (int j0 = 0; j0 < k; j0 += 8) {
     f32x4_a4 v[8];
 #pragma unroll

@@ -88,6 +88,9 @@ CASES = {
                                dict(gate_quant=J.Q8_0, down_quant=J.Q4_0)),
     "qwen3_30b_a3b_layers_q8_0": (QWEN3_MOE, (128, 8, 768, False), None, 256, 100, 2,
                                   dict(gate_quant=J.Q8_0, down_quant=J.Q8_0)),
+    # more than 128 experts beside a shared one: the combine kernel sums onto the shared expert's
+    # output and adds that to the residual
+    "shared_expert_of_256": (SMALL, (256, 8, 256, True), None, 128, 0, 4, {}),
 }
 
 
