@@ -241,6 +241,11 @@ int jero_hip_forward_model_forward(jero_forward_model *model, const uint32_t *to
  * n + max_tokens - 1 positions past max_positions ContextLengthExceeded.  Synchronous. */
 int jero_hip_forward_model_evaluate(jero_forward_model *model, const uint32_t *prompt, int64_t n, int64_t max_tokens,
                                     uint32_t *generated, float *timing_ms, void *stream);
+/* How the model's last evaluate ran its decode steps (the tokens are the same either way): NONE (no
+ * evaluate yet, or max_tokens 0), LAUNCH (all in one launch), GRAPH (a captured graph of launches);
+ * -1 for a null model. */
+enum { JERO_FWD_DECODE_NONE = 0, JERO_FWD_DECODE_LAUNCH = 1, JERO_FWD_DECODE_GRAPH = 2 };
+int jero_hip_forward_model_decode_form(const jero_forward_model *model);
 
 /* Load-time re-layout of a weight tensor for the GEMV kernels; replaces repack_tensor_parallel
  * (src/weights.rs:914-955) -> RepackedWeight.  Q4_K -> JERO_Q4_K_R and Q6_K -> JERO_Q6_K_R:

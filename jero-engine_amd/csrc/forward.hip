@@ -747,6 +747,7 @@ struct jero_forward_model {
   DecXch* xch = nullptr;
   int8_t* own = nullptr;
   uint32_t xtag = 0;
+  int form = JERO_FWD_DECODE_NONE;  // how the last evaluate ran its decode steps
 };
 
 namespace {
@@ -897,11 +898,12 @@ int capture_decode(jero_forward_model* f, int64_t n, int64_t max_tokens) {
   return JERO_OK;
 }
 
-// evaluate's decode steps as one launch of fwd_decode_kernel on gs; false, with nothing launched,
-// where the graph takes them: no buffers, more positions or head rows than it is made for, or a
-// device that refuses the cooperative launch.
-bool launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens) {
-  if (!f->xch || max_tokens < 2 || n + max_tokens - 1 > kDecPos) return false;
+// evaluate's decode steps as one launch of fwd_decode_kernel on gs; *launched false, with nothing
+// enqueued, where the graph takes them: no buffers, more positions or head rows than it is made for,
+// or a device that has no cooperative launch or no room for this one.
+int launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens, bool* launched) {
+  *launched = false;
+  if (!f->xch || max_tokens < 2 || n + max_tokens - 1 > kDecPos) return JERO_OK;
   DecArgs a{};
   for (int l = 0; l < kFwdLayers; l++) {
     for (int j = 0; j < kFwdMats; j++) a.w[l][j] = f->w[l][j];
@@ -912,13 +914,15 @@ bool launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens) {
   a.n = int(n), a.max_tokens = int(max_tokens), a.vocab = int(f->vocab), a.head_rows = int(f->head_rows);
   a.tag = f->xtag, a.seed = f->seed;
   void* args[] = {&a};
-  if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fwd_decode_kernel), dim3(kDecWgs), dim3(kMvWaves * 64),
-                                 args, 0, f->gs) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
+  const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fwd_decode_kernel), dim3(kDecWgs),
+                                                  dim3(kMvWaves * 64), args, 0, f->gs);
+  if (e != hipSuccess) (void)hipGetLastError();
+  if (e == hipErrorNotSupported || e == hipErrorCooperativeLaunchTooLarge) return JERO_OK;
+  const int rc = check_hip(e, "forward decode launch");
+  if (rc) return rc;
   f->xtag += uint32_t(kDecTags * (max_tokens - 1));
-  return true;
+  *launched = true;
+  return JERO_OK;
 }
 
 int check_model(const jero_forward_model* f, const char* who) {
@@ -966,18 +970,18 @@ extern "C" int jero_hip_forward_model_create(uint64_t seed, int64_t vocab, int64
   if (!rc && !(rc = fwd_alloc(f, size_t(f->head_rows) * kFwdDim, &p))) f->head = static_cast<int8_t*>(p);
   if (!rc && !(rc = fwd_alloc(f, size_t(f->head_rows) * sizeof(int32_t), &p))) f->logits = static_cast<int32_t*>(p);
   if (!rc && !(rc = fwd_alloc(f, cap * sizeof(uint32_t), &p))) f->tokens = static_cast<uint32_t*>(p);
-  // the one-launch decode's buffers (17 MB at most); without them evaluate replays a graph
+  // the one-launch decode's buffers (17 MB at most); where memory does not hold them evaluate replays
+  // a graph
   const size_t own_rows = std::min<size_t>(cap, kDecPos);
   if (!rc && f->head_rows <= kDecHeadRows) {
     void* px = nullptr;
     const size_t words = kDecCopies * sizeof(DecXch);
-    if (hipMalloc(&px, words + size_t(kDecWgs) * kFwdLayers * 2 * own_rows * kFwdDim) == hipSuccess &&
-        hipMemset(px, 0, words) == hipSuccess) {
+    const hipError_t e = hipMalloc(&px, words + size_t(kDecWgs) * kFwdLayers * 2 * own_rows * kFwdDim);
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (e != hipErrorOutOfMemory && !(rc = check_hip(e, "forward_model decode buffers"))) {
       f->owned.push_back(px);
       f->xch = static_cast<DecXch*>(px), f->own = static_cast<int8_t*>(px) + words;
-    } else {
-      (void)hipGetLastError();
-      (void)hipFree(px);
+      rc = check_hip(hipMemset(px, 0, words), "forward_model decode buffers");
     }
   }
   // ForwardModel::new (src/forward.rs:879-903): layer l's matrices from splitmix(seed ^ (16 l + j)),
@@ -1005,6 +1009,8 @@ extern "C" int jero_hip_forward_model_destroy(jero_forward_model* f) {
 extern "C" int64_t jero_hip_forward_model_head_rows(const jero_forward_model* f) { return f ? f->head_rows : -1; }
 
 extern "C" int64_t jero_hip_forward_model_positions(const jero_forward_model* f) { return f ? f->len : -1; }
+
+extern "C" int jero_hip_forward_model_decode_form(const jero_forward_model* f) { return f ? f->form : -1; }
 
 extern "C" int jero_hip_forward_model_reset(jero_forward_model* f) {
   if (!f) return fail(JERO_ERR_INVALID_ARGUMENT, "forward_model_reset: null model");
@@ -1073,12 +1079,14 @@ extern "C" int jero_hip_forward_model_evaluate(jero_forward_model* f, const uint
   if (!rc) rc = forward_rows(f, n, 0, f->logits, nullptr, s);
   if (!rc) rc = check_hip(hipEventRecord(ev[1], s), "event");
   // The decode steps run on the model's stream gs, after the prefill: in one launch where that takes
-  // the shape, else as one graph: the steps are
-  // the same launches for every evaluate of this (n, max_tokens), so they are captured once and
-  // replayed (the host then enqueues one graph instead of ~17 launches per token).
+  // the shape, else as one graph: the steps are the same launches for every evaluate of this
+  // (n, max_tokens), so they are captured once and replayed (the host then enqueues one graph instead
+  // of ~17 launches per token).
   if (!rc && !f->gs) rc = check_hip(hipStreamCreateWithFlags(&f->gs, hipStreamNonBlocking), "forward stream");
   if (!rc) rc = check_hip(hipStreamWaitEvent(f->gs, ev[1], 0), "forward stream order");
-  const bool one = !rc && launch_decode(f, n, max_tokens);
+  bool one = false;
+  if (!rc) rc = launch_decode(f, n, max_tokens, &one);
+  f->form = one ? JERO_FWD_DECODE_LAUNCH : max_tokens > 0 ? JERO_FWD_DECODE_GRAPH : JERO_FWD_DECODE_NONE;
   if (!rc && !one && max_tokens > 0 && (f->graph_n != n || f->graph_max != max_tokens || !f->graph))
     rc = capture_decode(f, n, max_tokens);
   if (!rc && !one && max_tokens > 0) rc = check_hip(hipGraphLaunch(f->graph, f->gs), "forward decode graph");

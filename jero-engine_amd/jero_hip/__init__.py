@@ -104,6 +104,7 @@ _SIGS = {
                                              C.POINTER(C.c_int)]),
     "jero_hip_forward_model_forward": (_I32, [_P, _P, _I64, _I64, _P, _P]),
     "jero_hip_forward_model_evaluate": (_I32, [_P, _P, _I64, _I64, _P, _P, _P]),
+    "jero_hip_forward_model_decode_form": (_I32, [_P]),
     "jero_hip_gguf_open": (_I32, [C.c_char_p, C.POINTER(_P)]),
     "jero_hip_gguf_close": (None, [_P]),
     "jero_hip_gguf_info": (_I32, [_P, C.POINTER(_I64), C.POINTER(C.c_char_p)]),
@@ -749,6 +750,14 @@ class ForwardModel:
                                                     _stream(stream)))
         toks = [int(v) for v in out[:max_tokens]]
         return (toks, (float(ms[0]), float(ms[1]))) if timing else toks
+
+    DECODE_NONE, DECODE_LAUNCH, DECODE_GRAPH = 0, 1, 2
+
+    @property
+    def decode_form(self):
+        """How the last evaluate() ran its decode steps: DECODE_NONE, DECODE_LAUNCH (one launch) or
+        DECODE_GRAPH (a captured graph of launches)."""
+        return int(lib().jero_hip_forward_model_decode_form(self.h))
 
 
 class DecodeModel:

@@ -285,4 +285,5 @@ def test_forward_model_argument_errors():
     assert L.jero_hip_forward_model_reset(None) == INVALID
     assert L.jero_hip_forward_model_head_rows(None) == -1
     assert L.jero_hip_forward_model_positions(None) == -1
+    assert L.jero_hip_forward_model_decode_form(None) == -1
     assert L.jero_hip_forward_model_destroy(None) == 0

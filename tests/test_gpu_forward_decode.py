@@ -37,8 +37,11 @@ def test_evaluate_equals_forward(vocab, n, max_tokens):
     prompt = prompt_of(n, vocab, n)
     ref, want, logits = expect(99, vocab, cap, prompt, max_tokens)
     m = J.ForwardModel(99, vocab, cap)
+    assert m.decode_form == m.DECODE_NONE
+    launch = max_tokens > 1 and n + max_tokens - 1 <= 128 and vocab <= 4096
     for _ in range(2):  # the exchange's words carry on
         assert m.evaluate(prompt, max_tokens) == want
+        assert m.decode_form == (m.DECODE_LAUNCH if launch else m.DECODE_GRAPH)
     got = torch.empty_like(logits)
     ref.forward([want[-1]], n + max_tokens - 1, logits)
     m.forward([want[-1]], n + max_tokens - 1, got)
