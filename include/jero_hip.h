@@ -242,10 +242,19 @@ int jero_hip_forward_model_forward(jero_forward_model *model, const uint32_t *to
 int jero_hip_forward_model_evaluate(jero_forward_model *model, const uint32_t *prompt, int64_t n, int64_t max_tokens,
                                     uint32_t *generated, float *timing_ms, void *stream);
 /* How the model's last evaluate ran its decode steps (the tokens are the same either way): NONE (no
- * evaluate yet, or max_tokens 0), LAUNCH (all in one launch), GRAPH (a captured graph of launches);
- * -1 for a null model. */
-enum { JERO_FWD_DECODE_NONE = 0, JERO_FWD_DECODE_LAUNCH = 1, JERO_FWD_DECODE_GRAPH = 2 };
+ * evaluate yet, or max_tokens 0), LAUNCH (all in one launch), GRAPH (a captured graph of launches),
+ * TIMED_OUT (the launch's workgroups, which have to be resident together, waited in vain beside other
+ * work on the device, and the graph ran the steps); -1 for a null model. */
+enum {
+  JERO_FWD_DECODE_NONE = 0,
+  JERO_FWD_DECODE_LAUNCH = 1,
+  JERO_FWD_DECODE_GRAPH = 2,
+  JERO_FWD_DECODE_TIMED_OUT = 3
+};
 int jero_hip_forward_model_decode_form(const jero_forward_model *model);
+/* Reads (about 1 us each) that a wave of the one-launch decode spends waiting for the others in one
+ * step before it gives up; 2^20 unless set, 0: at once. */
+int jero_hip_forward_model_set_decode_polls(jero_forward_model *model, int polls);
 
 /* Load-time re-layout of a weight tensor for the GEMV kernels; replaces repack_tensor_parallel
  * (src/weights.rs:914-955) -> RepackedWeight.  Q4_K -> JERO_Q4_K_R and Q6_K -> JERO_Q6_K_R:

@@ -411,14 +411,18 @@ __global__ void __launch_bounds__(256) fwd_fill_kernel(uint64_t seed, int64_t va
 // copy of the K / V rows, which only it writes, those of the prompt from the caches, the newest row
 // from the exchange.  A step takes 36 us; what bounds it is the 17 exchanges (a store to memory and a
 // read of it, about 1.5 us).
-// All workgroups have to be resident: the launch is cooperative.  A wave that waits in vain for
-// kDecSpins reads stops publishing, so every wait ends, and token 2^32 - 1 reports it.
+// All workgroups have to be resident at once: the launch is cooperative, which assures that they fit an
+// idle device, not that they are not kept waiting by another stream's or process's long kernels.  So
+// every wait ends: a wave that has read its words in vain `polls` times in one step (about 1 us each)
+// gives up, and from then on neither waits nor publishes, which ends the others' waits in turn.  Token
+// 2^32 - 1 reports it, and evaluate runs the steps again as the graph.  (The count is renewed once a
+// step: renewed by each wait it cost 1.6 % in spilled scalars.)
 constexpr int kDecWgs = 32, kDecWaves = kDecWgs * kMvWaves;
 constexpr int kDecWords = kFwdDim / 4;     // words of a model row
 constexpr int kDecHeadRows = 4096;         // head rows (exchange words) at most
 constexpr int kDecPos = int(kAttInMax);    // positions at most
 constexpr int kDecTags = 4 * kFwdLayers + 1;  // exchanges per step
-constexpr int kDecSpins = 1 << 22;
+constexpr int kDecPolls = 1 << 20;  // a step: about a second
 constexpr int kDecCopies = 8;  // of every word
 static_assert(kDecWaves == kDecWords, "a wave owns one word of a model row");
 
@@ -435,17 +439,18 @@ struct DecArgs {
   DecXch* x;  // [kDecCopies]
   const int32_t* logits0;  // the prompt's logits
   uint32_t* toks;
-  int n, max_tokens, vocab, head_rows;
+  int n, max_tokens, vocab, head_rows, polls;
   uint32_t tag;
   uint64_t seed;
 };
 
 struct DecWait {
-  int left = kDecSpins;
+  int left;  // reads that this step may still make in vain; 0: given up
   __device__ __forceinline__ bool dead() const { return left <= 0; }
 };
 
-// v[j] = the payload of word lane + STRIDE j (clamped to the last of n), once all carry the tag.
+// v[j] = the payload of word lane + STRIDE j (clamped to the last of n), once all carry the tag; any
+// value in a wave that gave up.
 template <int NW, int STRIDE = 64>
 __device__ __forceinline__ void dec_read(const uint64_t* __restrict__ words, int n, uint32_t tag, uint32_t (&v)[NW],
                                          DecWait& W) {
@@ -604,7 +609,7 @@ __global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
   int8_t* const own = a.own + int64_t(blockIdx.x) * (2 * kFwdLayers) * own_row;
   DecXch& X0 = a.x[0];
   DecXch& X = a.x[blockIdx.x % kDecCopies];
-  DecWait W;
+  DecWait W{a.polls};
   uint32_t tag = a.tag;
   for (int i = 1;; i++) {
     DecRow<8> wq[3];
@@ -627,6 +632,7 @@ __global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
     }
     const int vmax = wave_max_i(bi == INT32_MAX ? INT32_MIN : bv);
     const uint32_t tok = uint32_t(wave_min_i(bi != INT32_MAX && bv == vmax ? bi : INT32_MAX));
+    if (!W.dead()) W.left = a.polls;
     if (gw == 0 && lane == 0) a.toks[i - 1] = W.dead() ? ~0u : tok;
     if (i == a.max_tokens) break;
     const int pos = a.n + i - 1;
@@ -747,6 +753,7 @@ struct jero_forward_model {
   DecXch* xch = nullptr;
   int8_t* own = nullptr;
   uint32_t xtag = 0;
+  int polls = kDecPolls;
   int form = JERO_FWD_DECODE_NONE;  // how the last evaluate ran its decode steps
 };
 
@@ -912,7 +919,7 @@ int launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens, bool* la
   a.head = f->head, a.own = f->own, a.own_rows = int(std::min<int64_t>(f->cap, kDecPos)), a.x = f->xch;
   a.logits0 = f->logits, a.toks = f->tokens;
   a.n = int(n), a.max_tokens = int(max_tokens), a.vocab = int(f->vocab), a.head_rows = int(f->head_rows);
-  a.tag = f->xtag, a.seed = f->seed;
+  a.tag = f->xtag, a.seed = f->seed, a.polls = f->polls;
   void* args[] = {&a};
   const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fwd_decode_kernel), dim3(kDecWgs),
                                                   dim3(kMvWaves * 64), args, 0, f->gs);
@@ -1012,6 +1019,13 @@ extern "C" int64_t jero_hip_forward_model_positions(const jero_forward_model* f)
 
 extern "C" int jero_hip_forward_model_decode_form(const jero_forward_model* f) { return f ? f->form : -1; }
 
+extern "C" int jero_hip_forward_model_set_decode_polls(jero_forward_model* f, int polls) {
+  if (!f) return fail(JERO_ERR_INVALID_ARGUMENT, "forward_model_set_decode_polls: null model");
+  if (polls < 0) return fail(JERO_ERR_INVALID_ARGUMENT, "forward_model_set_decode_polls: negative count");
+  f->polls = polls;
+  return JERO_OK;
+}
+
 extern "C" int jero_hip_forward_model_reset(jero_forward_model* f) {
   if (!f) return fail(JERO_ERR_INVALID_ARGUMENT, "forward_model_reset: null model");
   f->len = 0;
@@ -1087,17 +1101,26 @@ extern "C" int jero_hip_forward_model_evaluate(jero_forward_model* f, const uint
   bool one = false;
   if (!rc) rc = launch_decode(f, n, max_tokens, &one);
   f->form = one ? JERO_FWD_DECODE_LAUNCH : max_tokens > 0 ? JERO_FWD_DECODE_GRAPH : JERO_FWD_DECODE_NONE;
-  if (!rc && !one && max_tokens > 0 && (f->graph_n != n || f->graph_max != max_tokens || !f->graph))
-    rc = capture_decode(f, n, max_tokens);
-  if (!rc && !one && max_tokens > 0) rc = check_hip(hipGraphLaunch(f->graph, f->gs), "forward decode graph");
-  if (!rc) rc = check_hip(hipEventRecord(ev[2], f->gs), "event");
-  if (!rc && max_tokens > 0)
-    rc = check_hip(hipMemcpyAsync(generated, toks, size_t(max_tokens) * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                  f->gs),
-                   "forward generated");
-  if (!rc) rc = check_hip(hipStreamSynchronize(f->gs), "forward_model_evaluate");
-  if (!rc && one && generated[max_tokens - 1] == ~0u)
-    rc = fail(JERO_ERR_DEVICE, "forward_model_evaluate: the decode launch's workgroups did not reach each other");
+  auto finish = [&]() {  // the decode's end and its tokens
+    int r = check_hip(hipEventRecord(ev[2], f->gs), "event");
+    if (!r && max_tokens > 0)
+      r = check_hip(hipMemcpyAsync(generated, toks, size_t(max_tokens) * sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                   f->gs),
+                    "forward generated");
+    return r ? r : check_hip(hipStreamSynchronize(f->gs), "forward_model_evaluate");
+  };
+  if (!rc && one) {
+    rc = finish();
+    // the workgroups did not meet within the limit: the prompt's logits and K / V rows, which the launch
+    // only reads, are still there for the graph
+    if (!rc && generated[max_tokens - 1] == ~0u) one = false, f->form = JERO_FWD_DECODE_TIMED_OUT;
+  }
+  if (!rc && !one) {
+    if (max_tokens > 0 && (f->graph_n != n || f->graph_max != max_tokens || !f->graph))
+      rc = capture_decode(f, n, max_tokens);
+    if (!rc && max_tokens > 0) rc = check_hip(hipGraphLaunch(f->graph, f->gs), "forward decode graph");
+    if (!rc) rc = finish();
+  }
   if (!rc && timing_ms) {
     rc = check_hip(hipEventElapsedTime(&timing_ms[0], ev[0], ev[1]), "event time");
     if (!rc) rc = check_hip(hipEventElapsedTime(&timing_ms[1], ev[1], ev[2]), "event time");

@@ -105,6 +105,7 @@ _SIGS = {
     "jero_hip_forward_model_forward": (_I32, [_P, _P, _I64, _I64, _P, _P]),
     "jero_hip_forward_model_evaluate": (_I32, [_P, _P, _I64, _I64, _P, _P, _P]),
     "jero_hip_forward_model_decode_form": (_I32, [_P]),
+    "jero_hip_forward_model_set_decode_polls": (_I32, [_P, _I32]),
     "jero_hip_gguf_open": (_I32, [C.c_char_p, C.POINTER(_P)]),
     "jero_hip_gguf_close": (None, [_P]),
     "jero_hip_gguf_info": (_I32, [_P, C.POINTER(_I64), C.POINTER(C.c_char_p)]),
@@ -751,13 +752,18 @@ class ForwardModel:
         toks = [int(v) for v in out[:max_tokens]]
         return (toks, (float(ms[0]), float(ms[1]))) if timing else toks
 
-    DECODE_NONE, DECODE_LAUNCH, DECODE_GRAPH = 0, 1, 2
+    DECODE_NONE, DECODE_LAUNCH, DECODE_GRAPH, DECODE_TIMED_OUT = 0, 1, 2, 3
 
     @property
     def decode_form(self):
-        """How the last evaluate() ran its decode steps: DECODE_NONE, DECODE_LAUNCH (one launch) or
-        DECODE_GRAPH (a captured graph of launches)."""
+        """How the last evaluate() ran its decode steps: DECODE_NONE, DECODE_LAUNCH (one launch),
+        DECODE_GRAPH (a captured graph of launches), or DECODE_TIMED_OUT (the launch's workgroups did
+        not meet, and the graph ran)."""
         return int(lib().jero_hip_forward_model_decode_form(self.h))
+
+    def set_decode_polls(self, polls):
+        """Reads that a wave of the one-launch decode spends waiting in one step before it gives up."""
+        check(lib().jero_hip_forward_model_set_decode_polls(self.h, polls))
 
 
 class DecodeModel:

@@ -286,4 +286,5 @@ def test_forward_model_argument_errors():
     assert L.jero_hip_forward_model_head_rows(None) == -1
     assert L.jero_hip_forward_model_positions(None) == -1
     assert L.jero_hip_forward_model_decode_form(None) == -1
+    assert L.jero_hip_forward_model_set_decode_polls(None, 1) == INVALID
     assert L.jero_hip_forward_model_destroy(None) == 0

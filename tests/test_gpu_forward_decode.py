@@ -50,6 +50,27 @@ def test_evaluate_equals_forward(vocab, n, max_tokens):
     assert torch.equal(got[:k], logits[:k])
 
 
+@pytest.mark.parametrize("vocab,n,max_tokens", [(1, 3, 5), (256, 11, 53), (4096, 5, 4)])
+def test_waits_in_vain_end_in_the_graph(vocab, n, max_tokens):
+    """With no read allowed every wave gives up at once (and leaves the kernel normally); with one a
+    step, most do.  Either way the tokens and the caches are those of the graph, and a later evaluate
+    runs in one launch again."""
+    cap = n + max_tokens
+    prompt = prompt_of(n, vocab, n)
+    ref, want, logits = expect(99, vocab, cap, prompt, max_tokens)
+    ref.forward([want[-1]], n + max_tokens - 1, logits)
+    m = J.ForwardModel(99, vocab, cap)
+    got = torch.empty_like(logits)
+    for polls, forms in ((0, [m.DECODE_TIMED_OUT]), (1, [m.DECODE_TIMED_OUT, m.DECODE_LAUNCH]),
+                         (1 << 20, [m.DECODE_LAUNCH]), (0, [m.DECODE_TIMED_OUT]), (1 << 20, [m.DECODE_LAUNCH])):
+        m.set_decode_polls(polls)
+        assert m.evaluate(prompt, max_tokens) == want, polls
+        assert m.decode_form in forms, polls
+        m.forward([want[-1]], n + max_tokens - 1, got)
+        torch.cuda.synchronize()
+        assert torch.equal(got[:max(vocab, 1)], logits[:max(vocab, 1)]), polls
+
+
 def test_shapes_in_turn_and_two_threads():
     shapes = [(11, 20), (3, 40), (30, 2)]
     want = [expect(5, 256, 64, prompt_of(i, 256, n), k)[1] for i, (n, k) in enumerate(shapes)]
