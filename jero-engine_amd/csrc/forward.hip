@@ -907,10 +907,15 @@ int capture_decode(jero_forward_model* f, int64_t n, int64_t max_tokens) {
 
 // evaluate's decode steps as one launch of fwd_decode_kernel on gs; *launched false, with nothing
 // enqueued, where the graph takes them: no buffers, more positions or head rows than it is made for,
-// or a device that has no cooperative launch or no room for this one.
+// a long prompt before a large head, or a device that has no cooperative launch or no room for this one.
+// Both grow in the one launch faster than in the graph's: past 64 positions every workgroup attends to
+// a second block of rows, and every wave reads all logits (graph and one launch, us: 4096 rows, prompt
+// 64, 64 steps 4204 and 4120, prompt 100, 28 steps 2128 and 2171; 3072 rows, prompt 120, 8 steps 940 and
+// 949; 2048 rows, prompt 100, 28 steps 2090 and 1964, prompt 120, 8 steps 926 and 917).
 int launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens, bool* launched) {
   *launched = false;
   if (!f->xch || max_tokens < 2 || n + max_tokens - 1 > kDecPos) return JERO_OK;
+  if (n > 64 && f->head_rows > 2048) return JERO_OK;
   DecArgs a{};
   for (int l = 0; l < kFwdLayers; l++) {
     for (int j = 0; j < kFwdMats; j++) a.w[l][j] = f->w[l][j];

@@ -29,16 +29,18 @@ def prompt_of(seed, vocab, n):
 
 
 # one head row; several reads of the logits and passes of the head; the last position of the launch's
-# own rows (need = 128), one more (the graph), one prompt row, one or two K / V blocks, one token
+# own rows (need = 128), one more (the graph), one prompt row, one or two K / V blocks, one token; a
+# large head before and after a prompt of one K / V block
 @pytest.mark.parametrize("vocab,n,max_tokens", [(0, 1, 2), (1, 3, 5), (5, 2, 1), (256, 1, 128), (256, 1, 129), (300, 64, 65),
-                                                (777, 60, 8), (4096, 5, 4), (4097, 5, 4)])
+                                                (777, 60, 8), (4096, 5, 4), (4097, 5, 4), (4096, 64, 3),
+                                                (2049, 65, 3), (2048, 65, 3)])
 def test_evaluate_equals_forward(vocab, n, max_tokens):
     cap = n + max_tokens
     prompt = prompt_of(n, vocab, n)
     ref, want, logits = expect(99, vocab, cap, prompt, max_tokens)
     m = J.ForwardModel(99, vocab, cap)
     assert m.decode_form == m.DECODE_NONE
-    launch = max_tokens > 1 and n + max_tokens - 1 <= 128 and vocab <= 4096
+    launch = max_tokens > 1 and n + max_tokens - 1 <= 128 and vocab <= (4096 if n <= 64 else 2048)
     for _ in range(2):  # the exchange's words carry on
         assert m.evaluate(prompt, max_tokens) == want
         assert m.decode_form == (m.DECODE_LAUNCH if launch else m.DECODE_GRAPH)
