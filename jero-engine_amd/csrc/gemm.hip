@@ -1036,29 +1036,41 @@ int launch_gemm_laid(int laid, const void* w, int64_t n_in, int64_t n_out, const
   // tokens (64) 17.8 and 7.7, 512 (512) 21.2 and 13.3; 4096 -> 4096 128 (512) 20.7 and 15.0, 192 (768)
   // 23.2 and 20.8, 256 (1024) 25.6 and 25.0; 4096 -> 14336 32 (448) 21.0 and 15.6, 64 (896) 24.7 and
   // 25.3; 12288 -> 1024 512 (512) 43.4 and 29.7, 768 (768) 45.8 and 48.8; Q6_K_P 12288 -> 4096 37
-  // (256) 59.8 and 29.3, 128 (512) 59.9 and 46.7, 192 (768) 60.6 and 61.3.  Beside another launch
-  // that fills most of the GPU the fewer workgroups of the tiles hide better (attn_v of 512 tokens:
-  // a 1.46 ms prefill took 1.2 % longer).
+  // (256) 59.8 and 29.3, 128 (512) 59.9 and 46.7.  Beyond two tiles per CU only up to 192 tokens and
+  // where each 32-token tile's own pass over the records stays cheap (in MB of records: Q6_K_P 8192 ->
+  // 4096 192 tokens (768, 68) 39.9 and 39.1, 12288 -> 4096 (768, 101) 59.3 and 60.6, 12288 -> 8192 96
+  // (768, 203) 64.1 and 69.4; Q4_K_G 12288 -> 8192 96 (768, 63) 44.2 and 40.8, 14336 -> 8192 96 (768,
+  // 73) 49.7 and 50.7, 28672 -> 8192 96 (768, 147) 90.5 and 99.2) and there is K to split (256 -> 4096
+  // 192 tokens 5.4 and 6.0).  Beside another launch that fills most of the GPU the fewer workgroups of
+  // the tiles hide better (attn_v of 512 tokens: a 1.46 ms prefill took 1.2 % longer).
+  constexpr int64_t kKwRecordBytes = 70'000'000;
+  const bool q4 = laid == JERO_Q4_K_G;
   const int64_t cus = device_info().cus;
-  const int64_t kw_tiles = ((m + 31) / 32) * ((n_out + 31) / 32);
-  if (kw_tiles <= (m <= 192 ? 3 : 2) * cus && !(beside && m > 128)) {
+  const int64_t n_tiles = (n_out + 31) / 32, kw_tiles = ((m + 31) / 32) * n_tiles;
+  const bool third = m <= 192 && nb > 1 && n_tiles * nb * (q4 ? kQ4gRec : kQ6pRec) <= kKwRecordBytes;
+  if (kw_tiles <= (third ? 3 : 2) * cus && !(beside && m > 128)) {
     if (split_out) *split_out = false;
     const bool wide = kw_tiles <= cus;
     const dim3 grid{unsigned(kw_tiles)}, block(wide ? 512 : 256);
     const uint8_t* xb = static_cast<const uint8_t*>(xq);
     const uint8_t* wb = static_cast<const uint8_t*>(w);
     const int64_t xrb = row_bytes(JERO_Q8_K, n_in);
-    auto* const kernel = laid == JERO_Q4_K_G ? (wide ? gemm_laid_kw_kernel<true, 8> : gemm_laid_kw_kernel<true, 4>)
-                                             : (wide ? gemm_laid_kw_kernel<false, 8> : gemm_laid_kw_kernel<false, 4>);
+    auto* const kernel = q4 ? (wide ? gemm_laid_kw_kernel<true, 8> : gemm_laid_kw_kernel<true, 4>)
+                            : (wide ? gemm_laid_kw_kernel<false, 8> : gemm_laid_kw_kernel<false, 4>);
     hipLaunchKernelGGL(kernel, grid, block, 0, s, xb, xrb, wb, int(m), int(n_out), nb, y);
     return check_launch("gemm (few tokens)");
   }
   // A grid that fills at most half of two workgroups per CU splits K in two: over the grid for a
   // caller that adds the halves itself, or where the tiles would leave half of the CUs empty; else
   // within the workgroup, without the zeroed output and its atomics (512 tokens, us over the grid and
-  // within: Q4_K_G 4096 -> 4096 35.8 and 28.3, 1024 -> 4096 23.6 and 11.9, Q6_K_P 12288 -> 4096 91.0
-  // and 93.2; 256 tokens 12288 -> 4096, 128 tiles: 47.9 and 60.9).
-  const int split = nb < 2 || tiles > cus ? kSplitNone : y2 || 2 * tiles <= cus ? kSplitGrid : kSplitWg;
+  // within: Q4_K_G 4096 -> 4096 35.8 and 28.3, 1024 -> 4096 23.6 and 11.9; 256 tokens Q6_K_P 12288 ->
+  // 4096, 128 tiles: 47.9 and 60.9).  Long rows stay on the grid, whose workgroups reach the CUs that
+  // fewer tiles leave empty: the record stream is then what bounds them (320 tokens -> 4096, 160 tiles:
+  // Q6_K_P 6144 38.3 and 34.4, 8192 47.7 and 57.3, 12288 71.6 and 87.9; Q4_K_G 14336 66.7 and 66.7,
+  // 28672 123.0 and 130.4), Q6_K_P but for a whole round of tiles (512 tokens 8192 -> 4096 61.1 and 59.3,
+  // 12288 -> 4096 88.7 and 88.5).
+  const bool in_wg = nb <= (q4 ? 56 : 24) || (!q4 && 8 * tiles > 7 * cus);
+  const int split = nb < 2 || tiles > cus ? kSplitNone : y2 || 2 * tiles <= cus || !in_wg ? kSplitGrid : kSplitWg;
   if (split_out) *split_out = split == kSplitGrid && y2;
   const uint8_t* xb = static_cast<const uint8_t*>(xq);
   const uint8_t* wb = static_cast<const uint8_t*>(w);
@@ -1070,7 +1082,6 @@ int launch_gemm_laid(int laid, const void* w, int64_t n_in, int64_t n_out, const
     if (rc) return rc;
   }
   const dim3 grid(unsigned(split == kSplitGrid ? 2 * tiles : tiles)), block(split == kSplitWg ? 2 * kGpThreads : kGpThreads);
-  const bool q4 = laid == JERO_Q4_K_G;
   auto* const kernel =
       split == kSplitGrid ? (q4 ? gemm_laid_kernel<true, kSplitGrid> : gemm_laid_kernel<false, kSplitGrid>)
       : split == kSplitWg ? (q4 ? gemm_laid_kernel<true, kSplitWg> : gemm_laid_kernel<false, kSplitWg>)

@@ -1,7 +1,7 @@
 """The GEMM's few-token form (K split over a workgroup's waves) and the Q4_K kernel at rows that are not
 a multiple of its tile, against one GEMV per row (held to the oracle by the GEMV tests).  Both sum
 the same exact block terms in f32 in another order: nb terms of at most the row's magnitude differ
-by a few nb * 2^-24, below 1e-5 of it for the 48 blocks here."""
+by a few nb * 2^-24, below 1e-5 of it for the 57 blocks here at most."""
 import numpy as np
 import pytest
 import torch
@@ -34,6 +34,16 @@ def check(quant, laid, m, n_in, n_out):
 @pytest.mark.parametrize("n_in", [256, 1792, 2304, 12288])  # fewer blocks than waves; ragged runs
 @pytest.mark.parametrize("quant", [J.Q4_K, J.Q6_K])
 def test_few_tokens(quant, n_in, m, n_out):
+    check(quant, True, m, n_in, n_out)
+
+
+# both sides of the rules between the forms: one block of K (two and more tiles per CU), records of 68
+# and 72 MB, and K halves within the workgroup or over the grid by the row's length and the tiles
+@pytest.mark.parametrize("quant,n_in,m,n_out", [
+    (J.Q4_K, 256, 128, 4096), (J.Q4_K, 256, 129, 4096), (J.Q6_K, 256, 97, 8192), (J.Q6_K, 8192, 161, 4096),
+    (J.Q6_K, 8704, 161, 4096), (J.Q4_K, 14336, 129, 4096), (J.Q6_K, 6144, 257, 4096), (J.Q6_K, 6400, 257, 4096),
+    (J.Q6_K, 6400, 449, 4096), (J.Q4_K, 14592, 257, 4096)])
+def test_rule_edges(quant, n_in, m, n_out):
     check(quant, True, m, n_in, n_out)
 
 
