@@ -1148,10 +1148,15 @@ using namespace jero;
 
 namespace jero {
 
-// Rows from which a Q4_K tensor whose rows are not a multiple of the tile runs the MFMA kernel rather
-// than one GEMV per row (4096 -> 1056: 8 rows 19 us as GEMVs and 27 here, 16 rows 37 and 27, 256 rows
-// 554 and 28; 2048 -> 5024: 8 rows 24 and 17).
-constexpr int64_t kRaggedMinRows = 16;
+// Activation rows from which a Q4_K tensor whose rows are not a multiple of the tile runs the MFMA
+// kernel rather than one GEMV per row.  The kernel's time is the serial chain of a row's blocks, whatever
+// the rows; a GEMV's is its launch and, from 2048 weight rows on, the weights (us as 16 GEMVs and here:
+// 4096 -> 1056 37 and 27, 5120 -> 31 34.1 and 30.4, 12288 -> 2080 76 and 66; 256 rows 4096 -> 1056 554
+// and 28).  Few and long weight rows take more of them (Q4_K_R -> 1000: 8192 20 rows 45.7 and 47.7, 24
+// 54.8 and 47.5; 12288 24 rows 64.2 and 68.9, 28 75.2 and 69.1; 28672 36 rows 198 and 154).
+int64_t ragged_min_rows(int64_t nb, int64_t n_out) {
+  return n_out >= 2048 || nb <= 20 ? 16 : std::min<int64_t>(nb / 2 + 6, 40);
+}
 
 int launch_gemm(int quant, const void* w_dev, int64_t n_in, int64_t n_out, const void* xq_dev, int64_t m, float* y_dev,
                 hipStream_t s, const void* laid, float* y2, bool* split_out, bool beside) {
@@ -1169,7 +1174,7 @@ int launch_gemm(int quant, const void* w_dev, int64_t n_in, int64_t n_out, const
     if (rc) return rc;
     return launch_gemm_laid(JERO_Q6_K_P, ws, n_in, n_out, xq_dev, m, y_dev, s);
   }
-  if ((quant == JERO_Q4_K || quant == JERO_Q4_K_R) && (n_out % kGemmBN == 0 || m >= kRaggedMinRows)) {
+  if ((quant == JERO_Q4_K || quant == JERO_Q4_K_R) && (n_out % kGemmBN == 0 || m >= ragged_min_rows(n_in / 256, n_out))) {
     const int tiles = gemm_tiles(m, n_out);
     const int nb = int(n_in / 256);
     // at most half the CUs busy (one 115 KB workgroup per CU): two workgroups per tile, one per

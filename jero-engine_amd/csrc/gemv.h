@@ -37,7 +37,7 @@ int launch_matvec(int quant, const void* w, int64_t n_in, int64_t n_out, const v
 // (w in that GEMM layout), or Q4_K / Q4_K_R / Q6_K / Q6_K_R with their GEMM layout given
 // (laid), run the int8-MFMA kernel over the layout; Q6_K / Q6_K_R from kLaidMinRows rows build
 // the Q6_K_P planes into the library workspace for the call; Q4_K / Q4_K_R run the int8-MFMA kernel
-// over the Q4_K bytes (n_out not a multiple of 128: from 16 rows on); one GEMV per row otherwise.
+// over the Q4_K bytes (n_out not a multiple of 128: from 16 to 40 rows on); one GEMV per row otherwise.
 // With y2 given, a layout GEMM whose grid splits K in two writes one half's sums to y and the other's to y2
 // (*split_out true; the product is y + y2, the same bits as the one-output form) instead of adding
 // both into a zeroed y.  beside: the launch runs on a second stream beside one that fills the GPU.

@@ -48,16 +48,17 @@ def test_rule_edges(quant, n_in, m, n_out):
 
 
 @pytest.mark.parametrize("laid_rows", [False, True])
-@pytest.mark.parametrize("m,n_out", [(15, 96), (16, 96), (17, 31), (130, 1000), (129, 4100)])
-def test_ragged_rows(m, n_out, laid_rows):
+@pytest.mark.parametrize("m,n_out,n_in", [(15, 96, 1024), (16, 96, 1024), (17, 31, 1024), (130, 1000, 1024),
+                                          (129, 4100, 1024), (29, 96, 12288), (30, 96, 12288), (16, 2080, 12288)])
+def test_ragged_rows(m, n_out, n_in, laid_rows):
     if laid_rows:
         dev = torch.device("cuda", 0)
-        w = J.TensorView("w", J.Q4_K, [1024, n_out], torch.from_numpy(rand_weights(J.Q4_K, n_out, 1024, 5)).to(dev))
-        x = J.quantize_act(J.Q8_K, torch.from_numpy(rand_act(m * 1024, m)).view(m, 1024).to(dev))
+        w = J.TensorView("w", J.Q4_K, [n_in, n_out], torch.from_numpy(rand_weights(J.Q4_K, n_out, n_in, 5)).to(dev))
+        x = J.quantize_act(J.Q8_K, torch.from_numpy(rand_act(m * n_in, m)).view(m, n_in).to(dev))
         a, b = torch.empty(m, n_out, device=dev), torch.empty(m, n_out, device=dev)
         J.gemm(w, x, m, a)
         J.gemm(J.repack(w), x, m, b)
         torch.cuda.synchronize()
         assert torch.equal(a, b)
     else:
-        check(J.Q4_K, False, m, 1024, n_out)
+        check(J.Q4_K, False, m, n_in, n_out)
