@@ -37,6 +37,18 @@ def test_one_launch_equals_two(quant, laid, n_out):
         assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), n_in
 
 
+# rows beyond 4096 elements run fused where the workgroups of 16 (or 8) rows leave no short last round
+# of the 256 CUs: from 4096 outputs, at whole rounds, and at 500 workgroups with a partial last one
+@pytest.mark.parametrize("n_out", [4096, 7999])
+@pytest.mark.parametrize("quant,laid,rows", [
+    (J.Q4_K, False, [4352, 7936]), (J.Q4_K, True, [4352, 6400, 8192]), (J.Q6_K, True, [4352, 5120]),
+    (J.Q8_0, False, [4128, 6176, 8192]), (J.Q4_0, False, [4128, 7168, 8192])])
+def test_long_rows(quant, laid, rows, n_out):
+    for n_in in rows:
+        y, ref = both(quant, laid, n_in, n_out)
+        assert np.array_equal(y.view(np.uint32), ref.view(np.uint32)), n_in
+
+
 @pytest.mark.parametrize("quant,n_in,n_out", [(J.Q4_K, 256, 25000), (J.Q8_0, 128, 400000), (J.Q4_K, 2304, 24577)])
 def test_many_rows(quant, n_in, n_out):
     y, ref = both(quant, False, n_in, n_out)
