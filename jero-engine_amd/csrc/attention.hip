@@ -1441,8 +1441,8 @@ static int attention_impl(AttnParams p, bool fused, int S, int T, float* out, in
   }
   // One split (up to 64 positions): the partial kernel divides its sums and writes the rows, without
   // the merge (one token, 32 heads of 128 over 8 KV heads, 1 / 64 positions: 7.5 / 7.8 us with it and
-  // 4.7 / 5.1 without).  The decode step's rings have more than one split.  An output that overlaps an input keeps the merge, which writes it after
-  // every workgroup has read.
+  // 4.7 / 5.1 without).  The decode step's rings have more than one split.  An output that overlaps an
+  // input keeps the merge, which writes it after every workgroup has read.
   const int64_t rows = int64_t(T) * nq * p.hd * int64_t(sizeof(float));
   const int64_t kv = int64_t(p.active) * p.nkv * p.hd * (p.kv_dtype == JERO_KV_F16 ? 2 : 4);
   auto meets = [&](const void* x, int64_t n) {

@@ -1302,7 +1302,8 @@ __global__ void __launch_bounds__(256, mfma_min_wgs(F, GU, PT)) moe_mfma_kernel(
 // r[t] = (accumulate ? y[t] : 0) + sum_j w[t, j] yd[inv[t, j]] in selection order, into y[t], or added
 // to resid[t] when given (y then only read).  Four outputs per thread and per_token workgroups to a
 // token, whose rows and weights are uniform loads: the rows' loads go out in eights before the first
-// sum.  One output per thread, each row's load waiting for its index, took 16.5 us at 512 tokens x 8 x 2048 (33 MB read) against 8.6.  H % 4 == 0 (the experts' is H % 256).
+// sum.  One output per thread, each row's load waiting for its index, took 16.5 us at 512 tokens x 8 x
+// 2048 (33 MB read) against 8.6.  H % 4 == 0 (the experts' is H % 256).
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ void __launch_bounds__(256) moe_combine_kernel(const float* __restrict__ yd, const float* __restrict__ w,
                                                           const int32_t* __restrict__ inv, int k, int H,

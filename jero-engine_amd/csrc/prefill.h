@@ -27,7 +27,7 @@ int launch_swiglu_rows(const float* g, int64_t g_stride, const float* u, int64_t
 int launch_add_rows(float* x, const float* d, const float* d2, int64_t count, hipStream_t s);
 // Per row t < n: X[t] += D[t] (+ D2[t], summed first, when given) when D is given, then the Q8_K
 // blocks of RMSNorm(X[t]) * w into Q (rows of H / 256 blocks), by the operations of launch_add_rows,
-// launch_rmsnorm_rows and launch_quantize_act (the norm within its last place); XN[t] (when given)
+// launch_rmsnorm_rows and launch_quantize_act (at some H the norm's scale within its last place); XN[t] (when given)
 // receives the normalised row.  H % 256 == 0, H <= 8192.
 int launch_add_rmsnorm_q8k_rows(float* X, const float* D, const float* D2, int64_t n, int64_t H, const float* w,
                                 float eps, float* XN, void* Q, hipStream_t s);
