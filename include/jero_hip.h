@@ -241,6 +241,9 @@ int jero_hip_forward_model_forward(jero_forward_model *model, const uint32_t *to
  * n + max_tokens - 1 positions past max_positions ContextLengthExceeded.  Synchronous. */
 int jero_hip_forward_model_evaluate(jero_forward_model *model, const uint32_t *prompt, int64_t n, int64_t max_tokens,
                                     uint32_t *generated, float *timing_ms, void *stream);
+/* ForwardExec::rmsnorm (src/forward.rs:672-699) of m device rows of 512 int8 (8-byte aligned; m in
+ * 1..2^22): y = clamp(48 x / max(isqrt(mean(x^2)), 1), -127, 127), truncating.  Enqueued on stream. */
+int jero_hip_forward_rmsnorm(const int8_t *x_dev, int64_t m, int8_t *out_dev, void *stream);
 /* How the model's last evaluate ran its decode steps (the tokens are the same either way): NONE (no
  * evaluate yet, or max_tokens 0), LAUNCH (all in one launch), GRAPH (a captured graph of launches),
  * TIMED_OUT (the launch's workgroups, which have to be resident together, waited in vain beside other

@@ -1022,6 +1022,16 @@ extern "C" int64_t jero_hip_forward_model_head_rows(const jero_forward_model* f)
 
 extern "C" int64_t jero_hip_forward_model_positions(const jero_forward_model* f) { return f ? f->len : -1; }
 
+extern "C" int jero_hip_forward_rmsnorm(const int8_t* x_dev, int64_t m, int8_t* out_dev, void* stream) {
+  if (!x_dev || !out_dev) return fail(JERO_ERR_INVALID_ARGUMENT, "forward_rmsnorm: null pointer");
+  if (m < 1 || m > kFwdMaxPositions) return fail(JERO_ERR_TENSOR_BOUNDS, "forward_rmsnorm: m must be in 1..2^22");
+  if ((reinterpret_cast<uintptr_t>(x_dev) | reinterpret_cast<uintptr_t>(out_dev)) & 7u)
+    return fail(JERO_ERR_INVALID_ARGUMENT, "forward_rmsnorm: rows must be 8-byte aligned");
+  hipLaunchKernelGGL(fwd_rmsnorm_rows_kernel, dim3(unsigned(m)), dim3(64), 0, static_cast<hipStream_t>(stream), x_dev,
+                     out_dev);
+  return check_launch("forward rmsnorm");
+}
+
 extern "C" int jero_hip_forward_model_decode_form(const jero_forward_model* f) { return f ? f->form : -1; }
 
 extern "C" int jero_hip_forward_model_set_decode_polls(jero_forward_model* f, int polls) {

@@ -104,6 +104,7 @@ _SIGS = {
                                              C.POINTER(C.c_int)]),
     "jero_hip_forward_model_forward": (_I32, [_P, _P, _I64, _I64, _P, _P]),
     "jero_hip_forward_model_evaluate": (_I32, [_P, _P, _I64, _I64, _P, _P, _P]),
+    "jero_hip_forward_rmsnorm": (_I32, [_P, _I64, _P, _P]),
     "jero_hip_forward_model_decode_form": (_I32, [_P]),
     "jero_hip_forward_model_set_decode_polls": (_I32, [_P, _I32]),
     "jero_hip_gguf_open": (_I32, [C.c_char_p, C.POINTER(_P)]),
@@ -751,6 +752,11 @@ class ForwardModel:
                                                     _stream(stream)))
         toks = [int(v) for v in out[:max_tokens]]
         return (toks, (float(ms[0]), float(ms[1]))) if timing else toks
+
+    @staticmethod
+    def rmsnorm(x, out, stream=None):
+        """ForwardExec::rmsnorm (:672-699) of int8 device rows x [m, 512] into out."""
+        check(lib().jero_hip_forward_rmsnorm(_ptr(x), x.shape[0], _ptr(out), _stream(stream)))
 
     DECODE_NONE, DECODE_LAUNCH, DECODE_GRAPH, DECODE_TIMED_OUT = 0, 1, 2, 3
 

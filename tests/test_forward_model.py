@@ -60,8 +60,8 @@ def test_isqrt_is_floor_sqrt():
 
 
 def test_device_integer_shortcuts_are_exact():
-    """The device RMSNorm replaces isqrt's Newton loop and the per-element division by cheaper
-    exact forms; both claims are checked here over their whole domain."""
+    """The device RMSNorm replaces isqrt's Newton loop by a cheaper exact form, checked here over its
+    whole domain (the per-element quotient: tests/test_forward_norm_quotient.py)."""
     # floor(sqrt(v)) from any root within one of it, by one correction each way, over the mean
     # squares a row can have (v <= 128^2) and well beyond
     v = np.arange(0, 1 << 20, dtype=np.int64)
@@ -71,11 +71,6 @@ def test_device_integer_shortcuts_are_exact():
         r = np.where(r * r > v, r - 1, r)
         r = np.where((r + 1) * (r + 1) <= v, r + 1, r)
         assert (r == root).all(), off
-    # |a| / d for |a| <= 6144 = 128 * 48 and 2 <= d <= 128: the high word of |a| * ceil(2^32 / d)
-    a = np.arange(0, 6145, dtype=np.uint64)
-    for d in range(2, 129):
-        mul = np.uint64(0xFFFFFFFF // d + 1)
-        assert ((a * mul) >> np.uint64(32) == a // np.uint64(d)).all(), d
 
 
 # ---------------------------------------------------------------- rmsnorm
@@ -286,5 +281,8 @@ def test_forward_model_argument_errors():
     assert L.jero_hip_forward_model_head_rows(None) == -1
     assert L.jero_hip_forward_model_positions(None) == -1
     assert L.jero_hip_forward_model_decode_form(None) == -1
+    assert L.jero_hip_forward_rmsnorm(None, 1, logits, None) == INVALID
+    assert L.jero_hip_forward_rmsnorm(logits, 0, logits, None) == BOUNDS
+    assert L.jero_hip_forward_rmsnorm(C.c_void_p(12), 1, logits, None) == INVALID
     assert L.jero_hip_forward_model_set_decode_polls(None, 1) == INVALID
     assert L.jero_hip_forward_model_destroy(None) == 0
