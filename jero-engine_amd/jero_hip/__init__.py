@@ -158,7 +158,7 @@ def check(status):
 
 # Every pointer argument is a plain integer (the entry points' argtypes convert it), and the current
 # stream is read as its handle: a torch.cuda.Stream object per call cost as much as the launch's own
-# host work.
+# host work.  Torch has the handle only under private names; without them the object serves.
 _raw_stream = None
 
 
@@ -169,8 +169,9 @@ def _stream(stream=None):
     if _raw_stream is None:
         import torch
         torch.cuda.current_stream()  # the first use initializes torch's GPU state
-        _raw_stream = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
-    return _raw_stream[0](_raw_stream[1]())
+        get, device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+        _raw_stream = (lambda: get(device())) if get and device else lambda: torch.cuda.current_stream().cuda_stream
+    return _raw_stream()
 
 
 def _ptr(t):
