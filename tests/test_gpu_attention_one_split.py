@@ -4,7 +4,11 @@ import numpy as np
 import pytest
 import torch
 
+import decode_parity as DP
 import jero_hip as J
+import model_spec as MS
+import pyoracle as O
+from test_gpu_decode import make_gpu_model, prefill_kv
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +41,18 @@ def test_output_over_the_queries():
     J.gqa_causal_attention_f32(buf[128:], buf[:4096], k, v, 32, 8, 128, 40, 0.1)
     torch.cuda.synchronize()
     assert torch.equal(buf[128:], want)
+
+
+@pytest.mark.parametrize("nq,nkv,hd,kv_f16", [(8, 2, 64, False), (4, 2, 128, False), (8, 8, 32, False), (8, 2, 32, True)])
+def test_batch_of_queries(dev, nq, nkv, hd, kv_f16):
+    """A prompt whose queries all see at most one split of positions, on rings that the flash kernel does
+    not take: every query's row lands at its own place (each token against the oracle)."""
+    spec = dict(hidden=512, ffn=1024, n_layers=2, vocab=1000, nq=nq, nkv=nkv, hd=hd, eps=1e-6, theta=1e6)
+    cap, pos0, n = 128, 5, 40
+    t = MS.build(spec, seed=37)
+    m = make_gpu_model(spec, t, cap, J.KV_F16 if kv_f16 else J.KV_F32, True)
+    om = O.DecodeModel(spec, MS.oracle_tensors(t), cap)
+    kv = prefill_kv(m, om, spec, cap, pos0, 41, dev, kv_f16)
+    tokens = np.random.default_rng(hd).integers(0, spec["vocab"], size=n).tolist()
+    DP.run_prefill_traced(m, om, t, spec, kv, cap, pos0, tokens, kv_f16, dev, True)
+    m.close()
