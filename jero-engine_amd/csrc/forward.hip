@@ -416,7 +416,8 @@ __global__ void __launch_bounds__(256) fwd_fill_kernel(uint64_t seed, int64_t va
 // every wait ends: a wave that has read its words in vain `polls` times in one step (about 1 us each)
 // gives up, and from then on neither waits nor publishes, which ends the others' waits in turn.  Token
 // 2^32 - 1 reports it, and evaluate runs the steps again as the graph.  (The count is renewed once a
-// step: renewed by each wait it cost 1.6 % in spilled scalars.)
+// step and a constant but for a limit that the caller set, LIMIT: renewed by each wait it cost 2 %, as
+// an argument 0.6 %, scalars that spill.)
 constexpr int kDecWgs = 32, kDecWaves = kDecWgs * kMvWaves;
 constexpr int kDecWords = kFwdDim / 4;     // words of a model row
 constexpr int kDecHeadRows = 4096;         // head rows (exchange words) at most
@@ -444,16 +445,20 @@ struct DecArgs {
   uint64_t seed;
 };
 
+template <bool LIMIT>
 struct DecWait {
-  int left;  // reads that this step may still make in vain; 0: given up
+  const DecArgs& a;
+  int left = polls();  // reads that this step may still make in vain; 0: given up
+  __device__ __forceinline__ explicit DecWait(const DecArgs& a_) : a(a_) {}
+  __device__ __forceinline__ int polls() const { return LIMIT ? a.polls : kDecPolls; }
   __device__ __forceinline__ bool dead() const { return left <= 0; }
 };
 
 // v[j] = the payload of word lane + STRIDE j (clamped to the last of n), once all carry the tag; any
 // value in a wave that gave up.
-template <int NW, int STRIDE = 64>
+template <int STRIDE = 64, int NW, bool LIMIT>
 __device__ __forceinline__ void dec_read(const uint64_t* __restrict__ words, int n, uint32_t tag, uint32_t (&v)[NW],
-                                         DecWait& W) {
+                                         DecWait<LIMIT>& W) {
   const int lane = threadIdx.x & 63;
   while (W.left > 0) {
     uint64_t r[NW];
@@ -472,7 +477,8 @@ __device__ __forceinline__ void dec_read(const uint64_t* __restrict__ words, int
 }
 
 // The word (of the first copy) into every copy; called by whole waves.
-__device__ __forceinline__ void dec_write(uint64_t* word, uint32_t tag, uint32_t v, const DecWait& W) {
+template <bool LIMIT>
+__device__ __forceinline__ void dec_write(uint64_t* word, uint32_t tag, uint32_t v, const DecWait<LIMIT>& W) {
   const int c = threadIdx.x & 63;
   if (c < kDecCopies && !W.dead())
     __hip_atomic_store(word + c * (sizeof(DecXch) / sizeof(uint64_t)), (uint64_t(tag) << 32) | v, __ATOMIC_RELAXED,
@@ -600,6 +606,7 @@ __device__ __forceinline__ void dec_attend(const DecArgs& a, int l, const int8_t
   __syncthreads();
 }
 
+template <bool LIMIT>
 __global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
   __shared__ __attribute__((aligned(16))) DecSmem S;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, g = lane >> 4;
@@ -609,7 +616,7 @@ __global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
   int8_t* const own = a.own + int64_t(blockIdx.x) * (2 * kFwdLayers) * own_row;
   DecXch& X0 = a.x[0];
   DecXch& X = a.x[blockIdx.x % kDecCopies];
-  DecWait W{a.polls};
+  DecWait<LIMIT> W(a);
   uint32_t tag = a.tag;
   for (int i = 1;; i++) {
     DecRow<8> wq[3];
@@ -632,7 +639,7 @@ __global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
     }
     const int vmax = wave_max_i(bi == INT32_MAX ? INT32_MIN : bv);
     const uint32_t tok = uint32_t(wave_min_i(bi != INT32_MAX && bv == vmax ? bi : INT32_MAX));
-    if (!W.dead()) W.left = a.polls;
+    if (!W.dead()) W.left = W.polls();
     if (gw == 0 && lane == 0) a.toks[i - 1] = W.dead() ? ~0u : tok;
     if (i == a.max_tokens) break;
     const int pos = a.n + i - 1;
@@ -672,7 +679,7 @@ __global__ void __launch_bounds__(kMvWaves * 64) fwd_decode_kernel(DecArgs a) {
       {  // word t of q | k | v, and word 256 + t of the first two waves
         uint32_t one[1] = {0u}, two[2] = {0u, 0u};
         if (wv < 2) {
-          dec_read<2, 256>(X.qkv + 64 * wv, 3 * kDecWords, tag, two, W);
+          dec_read<256>(X.qkv + 64 * wv, 3 * kDecWords, tag, two, W);
           S.qkv[t] = two[0];
           S.qkv[256 + t] = two[1];
           reinterpret_cast<uint32_t*>(own_v + int64_t(pos) * kFwdDim)[t] = two[1];
@@ -926,7 +933,8 @@ int launch_decode(jero_forward_model* f, int64_t n, int64_t max_tokens, bool* la
   a.n = int(n), a.max_tokens = int(max_tokens), a.vocab = int(f->vocab), a.head_rows = int(f->head_rows);
   a.tag = f->xtag, a.seed = f->seed, a.polls = f->polls;
   void* args[] = {&a};
-  const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fwd_decode_kernel), dim3(kDecWgs),
+  auto* const kernel = f->polls == kDecPolls ? fwd_decode_kernel<false> : fwd_decode_kernel<true>;
+  const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(kDecWgs),
                                                   dim3(kMvWaves * 64), args, 0, f->gs);
   if (e != hipSuccess) (void)hipGetLastError();
   if (e == hipErrorNotSupported || e == hipErrorCooperativeLaunchTooLarge) return JERO_OK;

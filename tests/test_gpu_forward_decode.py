@@ -64,7 +64,7 @@ def test_waits_in_vain_end_in_the_graph(vocab, n, max_tokens):
     m = J.ForwardModel(99, vocab, cap)
     got = torch.empty_like(logits)
     for polls, forms in ((0, [m.DECODE_TIMED_OUT]), (1, [m.DECODE_TIMED_OUT, m.DECODE_LAUNCH]),
-                         (1 << 20, [m.DECODE_LAUNCH]), (0, [m.DECODE_TIMED_OUT]), (1 << 20, [m.DECODE_LAUNCH])):
+                         (1 << 19, [m.DECODE_LAUNCH]), (0, [m.DECODE_TIMED_OUT]), (1 << 20, [m.DECODE_LAUNCH])):
         m.set_decode_polls(polls)
         assert m.evaluate(prompt, max_tokens) == want, polls
         assert m.decode_form in forms, polls
